@@ -26,6 +26,33 @@ __global__ __launch_bounds__(256) void k_fill_zero(uint4* __restrict__ dst, size
     if (blockIdx.x == 0 && threadIdx.x < ntail) tail[threadIdx.x] = 0;
 }
 
+// Rows of `units` U-sized units from a buffer with row stride `ss` units to one
+// with row stride `ds`.  Bound by memory latency on one chunk of a transfer
+// (at most 16 MiB, a few microseconds at the copy rate).  The block is bx units
+// by 256 / bx rows, so short rows still fill whole waves.
+template <typename U>
+__global__ __launch_bounds__(256) void k_rows(U* __restrict__ dst, size_t ds, const U* __restrict__ src, size_t ss,
+                                              size_t units, size_t rows, int bx)
+{
+    const int tx = (int)threadIdx.x % bx, ty = (int)threadIdx.x / bx, by = 256 / bx;
+    const size_t ystep = (size_t)gridDim.y * by, xstep = (size_t)gridDim.x * bx;
+    for (size_t r = (size_t)blockIdx.y * by + ty; r < rows; r += ystep)
+        for (size_t x = (size_t)blockIdx.x * bx + tx; x < units; x += xstep) dst[r * ds + x] = src[r * ss + x];
+}
+
+template <typename U>
+hipError_t rows_launch(void* dst, size_t dstride, const void* src, size_t sstride, size_t row_bytes, size_t rows,
+                       hipStream_t st)
+{
+    const size_t units = row_bytes / sizeof(U);
+    int bx = 1;
+    while (bx < 256 && (size_t)bx < units) bx *= 2;
+    const size_t gx = std::min<size_t>((units + bx - 1) / bx, 1024), gy = (rows + 256 / bx - 1) / (256 / bx);
+    hipLaunchKernelGGL(k_rows<U>, dim3((unsigned)gx, (unsigned)std::min<size_t>(gy, 65535)), dim3(256), 0, st, (U*)dst,
+                       dstride / sizeof(U), (const U*)src, sstride / sizeof(U), units, rows, bx);
+    return hipGetLastError();
+}
+
 // Copy the 2D ring (cells outside [r, N-r)^2) of src into dst, element size esz.
 __global__ __launch_bounds__(256) void k_copy_ring2d(Sweep2D s, int esz)
 {
@@ -106,6 +133,20 @@ hipError_t launch_fill_zero(void* dst, size_t bytes, hipStream_t st)
     hipLaunchKernelGGL(k_fill_zero, dim3(copy_blocks(n16)), dim3(256), 0, st, (uint4*)dst, n16,
                        (uint8_t*)dst + n16 * 16, tail);
     return hipGetLastError();
+}
+
+// The widest unit that divides the row and both strides (the buffers are at
+// least 256-byte aligned).
+hipError_t launch_rows(void* dst, size_t dstride, const void* src, size_t sstride, size_t row_bytes, size_t rows,
+                       hipStream_t st)
+{
+    if (row_bytes == 0 || rows == 0) return hipSuccess;
+    const size_t a = row_bytes | dstride | sstride;
+    if (a % 16 == 0) return rows_launch<uint4>(dst, dstride, src, sstride, row_bytes, rows, st);
+    if (a % 8 == 0) return rows_launch<uint2>(dst, dstride, src, sstride, row_bytes, rows, st);
+    if (a % 4 == 0) return rows_launch<uint32_t>(dst, dstride, src, sstride, row_bytes, rows, st);
+    if (a % 2 == 0) return rows_launch<uint16_t>(dst, dstride, src, sstride, row_bytes, rows, st);
+    return rows_launch<uint8_t>(dst, dstride, src, sstride, row_bytes, rows, st);
 }
 
 size_t diff_blocks(size_t nrows) { return nrows < 2048 ? (nrows ? nrows : 1) : 2048; }

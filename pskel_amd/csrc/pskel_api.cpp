@@ -235,7 +235,12 @@ Sweep3D make_sweep3d(const pskel_grid_t* g, const void* src, void* dst, int radi
 // Host rows <-> device pitched rows.  Transfers go through two pinned staging
 // buffers used in turn: the host side of one chunk of rows (a copy or a storage
 // conversion, on several threads) overlaps the DMA of the previous chunk.
-// A pageable source would be copied by the runtime one pitched row at a time.
+// Rows whose bytes are no multiple of 4 cross the link packed, in one contiguous
+// copy, and a kernel spreads them to (or gathers them from) the pitched rows:
+// there the runtime's own pitched copy takes 7 us per row (an upload of 1000 x
+// 1503 u8: 7.3 ms, packed 0.09 ms; 150 x 243 x 211 bf16: 267 ms, packed 0.54 ms).
+// Rows of whole words it moves at the link's rate by itself (150 x 243 x 212
+// bf16: 0.55 ms either way), without the extra buffer.
 // ---------------------------------------------------------------------------
 constexpr size_t kStageBytes = size_t(16) << 20;
 
@@ -255,9 +260,16 @@ pskel_status_t ensure_stage(pskel_grid_t* g)
         g->stage[b] = nullptr;
     }
     g->stage_bytes = 0;
+    if (g->bounce) (void)hipFree(g->bounce);
+    g->bounce = nullptr;
     for (int b = 0; b < 2; ++b) {
         PSKEL_HIP(hipHostMalloc(&g->stage[b], want, hipHostMallocDefault));
         if (!g->stage_ev[b]) PSKEL_HIP(hipEventCreateWithFlags(&g->stage_ev[b], hipEventDisableTiming));
+    }
+    // without device memory for the packed rows, pitched copies still work
+    if (rb % 4 != 0 && hipMalloc(&g->bounce, want) != hipSuccess) {
+        g->bounce = nullptr;
+        (void)hipGetLastError();
     }
     g->stage_bytes = want;
     return PSKEL_OK;
@@ -268,6 +280,14 @@ hipError_t stage_copy(pskel_grid_t* g, void* dbuf, void* stage, size_t r0, size_
 {
     const size_t rb = row_cells(g) * g->elem, pb = g->pitch * g->elem;
     char* dev = (char*)dbuf + r0 * pb;
+    if (pb != rb && g->bounce) {
+        if (kind == hipMemcpyHostToDevice) {
+            const hipError_t e = hipMemcpyAsync(g->bounce, stage, n * rb, kind, g->stream);
+            return e == hipSuccess ? launch_rows(dev, pb, g->bounce, rb, rb, n, g->stream) : e;
+        }
+        const hipError_t e = launch_rows(g->bounce, rb, dev, pb, rb, n, g->stream);
+        return e == hipSuccess ? hipMemcpyAsync(stage, g->bounce, n * rb, kind, g->stream) : e;
+    }
     if (kind == hipMemcpyHostToDevice)
         return pb == rb ? hipMemcpyAsync(dev, stage, n * rb, kind, g->stream)
                         : hipMemcpy2DAsync(dev, pb, stage, rb, rb, n, kind, g->stream);
@@ -835,6 +855,7 @@ pskel_status_t pskel_grid_destroy(pskel_grid_t* g)
         if (g->stage[b]) (void)hipHostFree(g->stage[b]);
         if (g->stage_ev[b]) (void)hipEventDestroy(g->stage_ev[b]);
     }
+    if (g->bounce) (void)hipFree(g->bounce);
     if (g->d_partials) (void)hipFree(g->d_partials);
     if (g->d_res) (void)hipFree(g->d_res);
     if (g->ev0) (void)hipEventDestroy(g->ev0);
@@ -862,8 +883,9 @@ pskel_status_t pskel_grid_upload(pskel_grid_t* g, int32_t which, const void* hos
         // u8 grids run life, whose byte-parallel kernels count neighbours of 0/1 cells
         if (host_dtype != PSKEL_DTYPE_U8) return fail(PSKEL_ERR_INVALID_ARGUMENT, "u8 grid: host dtype must be U8");
         const uint8_t* c = (const uint8_t*)host;
-        for (size_t i = 0; i < n; ++i)
-            if (c[i] > 1) return fail(PSKEL_ERR_INVALID_ARGUMENT, "life cells must be 0 or 1");
+        uint8_t any = 0;  // the OR of 0/1 cells is 0 or 1 (no early exit: the loop vectorises)
+        for (size_t i = 0; i < n; ++i) any |= c[i];
+        if (any > 1) return fail(PSKEL_ERR_INVALID_ARGUMENT, "life cells must be 0 or 1");
     }
     if (host_dtype == g->storage) {
         if (g->auto_offset && which == PSKEL_BUFFER_INPUT)

@@ -227,6 +227,9 @@ hipError_t launch_reduce_partials(const double* partials, size_t n, double* out,
 // Utilities.
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t st);
 hipError_t launch_fill_zero(void* dst, size_t bytes, hipStream_t st);
+// rows of row_bytes between buffers of different row strides (bytes)
+hipError_t launch_rows(void* dst, size_t dstride, const void* src, size_t sstride, size_t row_bytes, size_t rows,
+                       hipStream_t st);
 hipError_t launch_copy_ring2d(const Sweep2D& s, int elem, hipStream_t st);
 
 }  // namespace pskel
@@ -245,6 +248,9 @@ struct pskel_grid : pskel::Grid {
     // in turn (allocated by the first transfer, at most 16 MiB each)
     void* stage[2] = {nullptr, nullptr};
     size_t stage_bytes = 0;
+    // device side of a chunk whose rows are packed on the host and pitched in
+    // the grid (stage_bytes; NULL: rows without padding, or no memory for it)
+    void* bounce = nullptr;
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
 };
 
