@@ -405,7 +405,7 @@ size_t diff_blocks(size_t nrows);
 namespace {
 
 struct RunPlan {
-    int path = 0;     // 0 plain, 1 tuned, 2 temporal
+    int path = 0;     // 0 plain, 1 tuned, 2 temporal, 3 any mask through an LDS tile (tuned)
     int pattern = PAT_GENERIC;
     int radius = 0;
 };
@@ -507,7 +507,8 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
                 else if (plan.path >= 1) e = launch_life_tuned(s, one, st);
                 else e = launch_life_plain(s, pts, bx, by, st);
             } else {
-                if (k > 1)
+                if (plan.path == 3) e = launch_2d_points_f32(s, pts, st);
+                else if (k > 1)
                     e = cfg.tile_x > 0 ? launch_2d_march_f32(s, pts, plan.pattern, (int)k, cfg, st)
                                        : launch_2d_ttile_f32(s, pts, plan.pattern, (int)k, cfg, st);
                 else if (plan.path >= 1) e = launch_2d_tuned_f32(s, pts, plan.pattern, one, st);
@@ -518,7 +519,10 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
             if (g->storage == PSKEL_DTYPE_BF16 || g->storage == PSKEL_DTYPE_F16)
                 s.c0 = scaled_sum_offset_term(pts.coeff, pts.np, g->store_offset);
             size_t nb;
-            if (k >= 2) {
+            if (plan.path == 3) {
+                nb = points3d_blocks(s, pts);
+                e = launch_3d_points(s, pts, g->storage, st);
+            } else if (k >= 2) {
                 nb = ttile3d_blocks(s, g->storage, cfg, (int)k);
                 e = launch_3d_ttile(s, pts, g->storage, cfg, (int)k, st);
             } else if (plan.path >= 1) {
@@ -649,7 +653,23 @@ pskel_status_t plan_run(const pskel_grid_t* g, const pskel_stencil_desc_t* d, co
                             "3D temporal tile shape (cells per lane, rows per wave, waves along d and w, depth)");
             plan.path = 2;
         }
-        if (!tunable) plan.path = 0;  // no specialised kernel for this point set: the plain kernel runs
+        if (!tunable) {
+            // no specialised kernel for this point set: the LDS tile of any
+            // mask, or the plain kernel where its halo does not fit and on
+            // small grids, whose few tiles leave the device idle.  Measured,
+            // plain / tile: 2D 512 x 512 3 points 3.5 / 4.8 us, 25 points 5.4 /
+            // 6.5; 800 x 1000 5.7 / 5.0 and 11.5 / 6.7; 3D 40^3 7 points 4.0 /
+            // 4.6, 13 points 7.0 / 5.4; 64^3 7 points 4.6 / 4.5
+            plan.path = 0;
+            Points pts;
+            fill_points(pts, *d, ndim);
+            const size_t n = cells(g);
+            const bool pays = ndim == 2 ? n >= 640 * 1024 : pts.np >= 8 || n >= 256 * 1024;
+            const bool tile = !pays ? false
+                              : ndim == 2 ? g->storage == PSKEL_DTYPE_F32 && points2d_ok((int)g->W, (int)g->H, pts)
+                                          : points3d_blocks(make_sweep3d(g, nullptr, nullptr, radius, nullptr), pts) > 0;
+            if (tile) plan.path = 3;
+        }
     }
     if (plan.path == 0) {
         // plain launches keep the caller's block; it must have whole waves when the
@@ -666,10 +686,13 @@ namespace {
 // FP64 partials a run with residuals needs: one per block of the largest
 // launch its sweeps use (3D sweeps reduce inside the stencil launch), or of
 // the separate difference kernel (2D).
-size_t residual_partials(const pskel_grid_t* g, const RunPlan& plan, const pskel_launch_cfg_t& cfg)
+size_t residual_partials(const pskel_grid_t* g, const RunPlan& plan, const Points& pts,
+                         const pskel_launch_cfg_t& cfg)
 {
     size_t nb = diff_blocks(g->nrows);
-    if (g->ndim == 3) {
+    if (g->ndim == 3 && plan.path == 3) {
+        nb = std::max(nb, points3d_blocks(make_sweep3d(g, nullptr, nullptr, plan.radius, nullptr), pts));
+    } else if (g->ndim == 3) {
         const int bx = cfg.block_x > 0 ? cfg.block_x : 64;
         const int by = cfg.block_y > 0 ? cfg.block_y : 4;
         Sweep3D s3 = make_sweep3d(g, nullptr, nullptr, plan.radius, nullptr);
@@ -998,7 +1021,7 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
     const size_t every = cfg.residual_every > 0 ? (size_t)cfg.residual_every : 0;
     const size_t nres_max = every ? iterations / every : 0;
     if (every) {
-        if ((st = ensure_partials(g, residual_partials(g, plan, cfg))) != PSKEL_OK) return st;
+        if ((st = ensure_partials(g, residual_partials(g, plan, pts, cfg))) != PSKEL_OK) return st;
         if ((st = ensure_res(g, nres_max)) != PSKEL_OK) return st;
     }
     if (plan.path == 2 && ndim == 3) {
@@ -1206,6 +1229,8 @@ extern "C" pskel_status_t pskel_run_iterative_noalloc(const pskel_grid_desc_t* d
     RunPlan plan;
     pskel_status_t st = plan_run(&g, d, cfg, plan);
     if (st != PSKEL_OK) return st;
+    Points pts;
+    fill_points(pts, *d, g.ndim);
     const size_t every = cfg.residual_every > 0 ? (size_t)cfg.residual_every : 0;
     const size_t nres = every ? iterations / every : 0;
     if (nres > kScratchResiduals)
@@ -1214,7 +1239,7 @@ extern "C" pskel_status_t pskel_run_iterative_noalloc(const pskel_grid_desc_t* d
     double* scr = nullptr;
     if ((st = scratch_of(desc->device, &scr)) != PSKEL_OK) return st;
     if (every) {
-        const size_t nb = residual_partials(&g, plan, cfg);
+        const size_t nb = residual_partials(&g, plan, pts, cfg);
         if (nb > kScratchPartials)
             return fail(PSKEL_ERR_INVALID_ARGUMENT, "residuals of launches of more than 65536 blocks need a grid");
         g.d_partials = scr;
@@ -1223,8 +1248,6 @@ extern "C" pskel_status_t pskel_run_iterative_noalloc(const pskel_grid_desc_t* d
         g.res_cap = kScratchResiduals;
     }
     hipStream_t stream = (hipStream_t)cfg.stream;  // NULL: the null stream
-    Points pts;
-    fill_points(pts, *d, g.ndim);
     int64_t nl = 0, nr = 0;
     if (iterations > 0 && (st = issue(&g, *d, pts, iterations, cfg, plan, stream, &nl, &nr)) != PSKEL_OK) return st;
     // the result goes to `out`, as runIterativeGPU leaves it in output

@@ -200,6 +200,12 @@ hipError_t launch_2d_march_f32(const Sweep2D& s, const Points& p, int pattern, i
 // a grid the register march takes: wider than 8 cells, buffer under 2 GiB
 bool march2d_ok(int W, int H, size_t pitch);
 
+// arbitrary masks through an LDS tile (k_points.hip): masks whose halo fits it
+bool points2d_ok(int W, int H, const Points& p);
+hipError_t launch_2d_points_f32(const Sweep2D& s, const Points& p, hipStream_t st);
+hipError_t launch_3d_points(const Sweep3D& s, const Points& p, int storage, hipStream_t st);
+size_t points3d_blocks(const Sweep3D& s, const Points& p);  // 0: the halo does not fit
+
 // 2D life (u8) sweeps.
 hipError_t launch_life_plain(const Sweep2D& s, const Points& p, int bx, int by, hipStream_t st);
 hipError_t launch_life_tuned(const Sweep2D& s, const pskel_launch_cfg_t& cfg, hipStream_t st);

@@ -147,6 +147,7 @@ std::vector<pskel_launch_cfg_t> candidates(const pskel_tune_query_t& q, const ps
         }
         v.push_back(plain(64, 4));
     } else {
+        v.push_back(tuned(0, 0, 0, 1));  // the LDS tile of any mask (the plain kernel where it does not fit)
         const int blocks[][2] = {{64, 1}, {64, 2}, {64, 4}, {128, 2}, {256, 1}, {32, 4}};
         for (auto& b : blocks) v.push_back(plain(b[0], b[1]));
     }
@@ -279,7 +280,9 @@ pskel_launch_cfg_t heuristic(const pskel_tune_query_t& q, const pskel_stencil_de
             }
         return tuned(vd, rw, hs, 1);
     }
-    return plain(64, 4);
+    // any other mask: the LDS tile (3D, 7 to 27 points: 2.5 to 10 times the plain
+    // kernel from 192 x 225 x 260 up, level with it or faster down to 60 x 70 x 50)
+    return tuned(0, 0, 0, 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -467,7 +470,8 @@ pskel_status_t pskel_tuner_choose(const pskel_mlp_t* model, const pskel_tune_que
         std::lock_guard<std::mutex> lock(g_predict_mutex);
         model = g_default_model;
     }
-    if (!model) {
+    // the model's training queries hold no masks without a specialised kernel
+    if (!model || classify(*d, q->ndim) == PAT_GENERIC) {
         *out = heuristic(*q, *d);
         return PSKEL_OK;
     }
