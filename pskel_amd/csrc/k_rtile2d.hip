@@ -1,0 +1,157 @@
+// Register tiles of the radius-1 2D stencils: launch plans and launches
+// (the kernel is k_rtile2d.hpp).
+#define PSKEL_RTILE_INSTANTIATE
+#include "k_rtile2d.hpp"
+
+namespace pskel {
+
+bool rtile2d_ok(int pattern, int W, int H, size_t pitch)
+{
+    // the register march (k_march2d.hpp) holds the 9-point stencil's large
+    // grids: both are at the VALU's rate there, and its waves overlap less
+    // (4096^2: march 11.5 us a sweep, tiles 11.9; 8192^2 36-39 against 39-44;
+    // 3000 x 3500 8.5 against 8.4; 2048^2 4.9 against 4.3)
+    if (pattern == PAT_BOX9 && (double)W * H > 12e6) return false;
+    return rt_fits(W, H, pitch);
+}
+
+// a tile outputs rows and columns after q.k sweeps
+static bool rt_depth_ok(int W, int H, const RtPlan& q)
+{
+    return q.k >= 1 && (H <= q.r * q.nw || 2 * q.k < q.r * q.nw) && (W <= kRtCols || 2 * rt_halo_cols(q.k) < kRtCols);
+}
+
+namespace {
+
+// Tile shapes and the blocks of each that a CU holds (registers, waves, LDS).
+struct RtShape {
+    int pattern, r, nw, per_cu;
+};
+constexpr RtShape kRtShapes[] = {
+    {PAT_J5, 2, 16, 2},   {PAT_J5, 4, 8, 4},    {PAT_J5, 4, 16, 2},   {PAT_J5, 8, 8, 3},
+    {PAT_BOX9, 2, 8, 4},  {PAT_BOX9, 2, 16, 2}, {PAT_BOX9, 4, 8, 4},  {PAT_BOX9, 4, 16, 2},
+    {PAT_CLOUD, 2, 8, 4}, {PAT_CLOUD, 2, 16, 2}, {PAT_CLOUD, 4, 8, 3},
+};
+
+// Time of one launch in microseconds: a launch, then rounds of blocks, each
+// sweep of a round at the VALU's rate for the rows a CU holds or, with few, at
+// the latency of a barrier and one block's rows; no less than its bytes take.
+// The constants are a least-squares fit of 820, 640 and 420 measured launches
+// (64^2 to 4096^2, depths 1 to 32): the fastest choice or one within 10% on 25
+// of 27 grids, 19% at worst.
+struct RtCost {
+    double launch, round, row, barrier, bytes;  // us, us, us per wave-row, us, bytes per us
+};
+constexpr RtCost rt_cost(int pattern)
+{
+    return pattern == PAT_J5     ? RtCost{3.30, 0.19, 0.0096, 0.272, 7.6e6}
+           : pattern == PAT_BOX9 ? RtCost{3.34, 0.00, 0.0269, 0.327, 6.2e6}
+                                 : RtCost{2.64, 1.39, 0.0316, 0.282, 7.2e6};
+}
+constexpr int kRtCus = 256;    // what the fit was measured on
+constexpr int kRtMaxDepth = 32;
+
+double rt_time(const RtShape& h, int W, int H, int k)
+{
+    const RtCost c = rt_cost(h.pattern);
+    const int rows = h.r * h.nw;
+    const int64_t nb = (int64_t)rt_tiles(W, kRtCols, rt_halo_cols(k)) * rt_tiles(H, rows, k);
+    const int64_t slots = (int64_t)kRtCus * h.per_cu, full = nb / slots, rest = nb % slots;
+    auto round = [&](int64_t b) {
+        return c.round + k * std::max(c.row * (double)(b * rows), c.barrier + c.row * rows);
+    };
+    const double t = c.launch + (double)full * round(h.per_cu) + (rest ? round((rest + kRtCus - 1) / kRtCus) : 0.0);
+    const double bytes = 4.0 * ((h.pattern == PAT_CLOUD ? 3.0 : 1.0) * (double)nb * kRtCols * rows + (double)W * H);
+    return std::max(t, c.launch + bytes / c.bytes);
+}
+
+}  // namespace
+
+// The shape and depth with the least time for the run's remaining sweeps, cut
+// into launches of equal depth.  An even depth keeps the state's ring in place
+// (the next launch needs no ring copy); an odd one may end the run.
+RtPlan rtile2d_plan(int pattern, int W, int H, size_t rem, bool odd)
+{
+    RtPlan best;
+    double best_t = 0.0;
+    for (const RtShape& h : kRtShapes) {
+        if (h.pattern != pattern) continue;
+        for (int k = 1; k <= kRtMaxDepth && (size_t)k <= rem; ++k) {
+            const RtPlan q{h.r, h.nw, k};
+            if (!rt_depth_ok(W, H, q)) break;
+            if ((size_t)k != rem && k != 1 && (k % 2 == 1) != odd) continue;
+            if (odd && k % 2 == 0) continue;
+            const double t = rt_time(h, W, H, k) * (double)((rem + k - 1) / k);
+            if (best.k && t >= best_t) continue;
+            best = q;
+            best_t = t;
+        }
+    }
+    // the same number of launches, evened out
+    const size_t n = (rem + best.k - 1) / best.k;
+    size_t k = (rem + n - 1) / n;
+    if (n > 1 && (k % 2 == 1) != odd) k += 1;
+    best.k = (int)std::min<size_t>(k, (size_t)best.k);
+    return best;
+}
+
+namespace {
+
+template <int PAT, int R, int NW>
+hipError_t rt_go(const Sweep2D& s, const RtParams& p, int k, double* partials, hipStream_t st)
+{
+    const int ntx = rt_tiles(s.W, kRtCols, rt_halo_cols(k)), nty = rt_tiles(s.H, R * NW, k);
+    const dim3 grid((unsigned)(ntx * nty)), block(NW * kWave);
+    if (partials) hipLaunchKernelGGL((k2d_rtile<PAT, R, NW, true>), grid, block, 0, st, s, p, ntx, k, partials);
+    else hipLaunchKernelGGL((k2d_rtile<PAT, R, NW, false>), grid, block, 0, st, s, p, ntx, k, partials);
+    return hipGetLastError();
+}
+
+template <int PAT>
+hipError_t rt_shape(const Sweep2D& s, const RtParams& p, const RtPlan& q, double* partials, hipStream_t st)
+{
+#define PSKEL_RT(R, NW) \
+    if (q.r == R && q.nw == NW) return rt_go<PAT, R, NW>(s, p, q.k, partials, st);
+    // the shapes of kRtShapes
+    PSKEL_RT(2, 16)
+    PSKEL_RT(4, 8)
+    if constexpr (PAT != PAT_J5) {
+        PSKEL_RT(2, 8)
+    }
+    if constexpr (PAT != PAT_CLOUD) {
+        PSKEL_RT(4, 16)
+    }
+    if constexpr (PAT == PAT_J5) {
+        PSKEL_RT(8, 8)
+    }
+#undef PSKEL_RT
+    return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+size_t rtile2d_blocks(int W, int H, const RtPlan& q)
+{
+    return (size_t)rt_tiles(W, kRtCols, rt_halo_cols(q.k)) * rt_tiles(H, q.r * q.nw, q.k);
+}
+
+hipError_t launch_2d_rtile(const Sweep2D& s, const Points& pts, const CloudArgs* cloud, int pattern, const RtPlan& q,
+                           double* partials, hipStream_t st)
+{
+    if (!rt_fits(s.W, s.H, s.pitch) || (partials && q.k != 1) || !rt_depth_ok(s.W, s.H, q)) return hipErrorInvalidValue;
+    RtParams p{};
+    p.coeff = pts.coeff;
+    for (int i = 0; i < 9; ++i) p.wt[i] = pts.wt[i];
+    if (cloud) {
+        p.coeff = cloud->dt;
+        p.wx = cloud->wx;
+        p.wy = cloud->wy;
+        p.fpitch = (uint32_t)cloud->fpitch;
+    }
+    if (pattern == PAT_J5) return rt_shape<PAT_J5>(s, p, q, partials, st);
+    if (pattern == PAT_BOX9) return rt_shape<PAT_BOX9>(s, p, q, partials, st);
+    if (pattern == PAT_CLOUD && cloud) return rt_shape<PAT_CLOUD>(s, p, q, partials, st);
+    return hipErrorInvalidValue;
+}
+
+}  // namespace pskel

@@ -408,6 +408,7 @@ struct RunPlan {
     int path = 0;     // 0 plain, 1 tuned, 2 temporal, 3 any mask through an LDS tile (tuned)
     int pattern = PAT_GENERIC;
     int radius = 0;
+    bool rtile = false;  // 2D fused sweeps on register tiles, as many per launch as pays
 };
 
 // Sweeps fused in the next launch: up to the temporal depth, cut so that a launch
@@ -418,14 +419,20 @@ struct RunPlan {
 // sweep short and the residual step runs as a single sweep.  A 2D launch of an
 // even number of sweeps writes a spare buffer; without one (odd2d) a launch
 // fuses one sweep less.
-size_t next_k(size_t done, size_t iterations, int kmax, size_t every, int ndim, bool odd2d)
+// On register tiles the launch is as deep as rtile2d_plan makes it (*rt).
+size_t next_k(const pskel::Grid& g, const RunPlan& plan, size_t done, size_t iterations, int kmax, size_t every,
+              RtPlan* rt)
 {
-    size_t k = std::min<size_t>((size_t)kmax, iterations - done);
+    size_t k = plan.rtile ? iterations - done : std::min<size_t>((size_t)kmax, iterations - done);
     if (every) {
         k = std::min(k, (done / every + 1) * every - done);
-        if (ndim == 2 && k > 1 && (done + k) % every == 0) k -= 1;
+        if (g.ndim == 2 && k > 1 && (done + k) % every == 0) k -= 1;
     }
-    if (odd2d && ndim == 2 && k % 2 == 0) k -= 1;
+    if (plan.rtile) {
+        *rt = rtile2d_plan(plan.pattern, (int)g.W, (int)g.H, k, g.odd_2d_launches);
+        return (size_t)rt->k;
+    }
+    if (g.odd_2d_launches && g.ndim == 2 && k % 2 == 0) k -= 1;
     return k;
 }
 
@@ -459,7 +466,8 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
     size_t done = 0;
     int64_t nl = 0, nr = 0;
     while (done < iterations) {
-        const size_t k = next_k(done, iterations, kmax, every, ndim, g->odd_2d_launches);
+        RtPlan rt;
+        const size_t k = next_k(*g, plan, done, iterations, kmax, every, &rt);
         const bool want_res = every && ((done + k) % every == 0);
         const void* src = g->buf[0];
         void* dst;
@@ -500,7 +508,8 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
                 field_info(g->fields[0], &fd, &fw, &fh, &fz, &ca.wx, &ca.fpitch);
                 field_info(g->fields[1], &fd, &fw, &fh, &fz, &ca.wy, &ca.fpitch);
                 ca.dt = d.coeff;
-                if (plan.path >= 1) e = launch_cloud_tuned(s, ca, one, st);
+                if (plan.rtile) e = launch_2d_rtile(s, pts, &ca, plan.pattern, rt, want_res ? g->d_partials : nullptr, st);
+                else if (plan.path >= 1) e = launch_cloud_tuned(s, ca, one, st);
                 else e = launch_cloud_plain(s, ca, bx, by, st);
             } else if (g->storage == PSKEL_DTYPE_U8) {
                 if (k > 1) e = launch_life_bits(s, (int)k, cfg, st);
@@ -508,11 +517,17 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
                 else e = launch_life_plain(s, pts, bx, by, st);
             } else {
                 if (plan.path == 3) e = launch_2d_points_f32(s, pts, st);
+                else if (plan.rtile)
+                    e = launch_2d_rtile(s, pts, nullptr, plan.pattern, rt, want_res ? g->d_partials : nullptr, st);
                 else if (k > 1)
                     e = cfg.tile_x > 0 ? launch_2d_march_f32(s, pts, plan.pattern, (int)k, cfg, st)
                                        : launch_2d_ttile_f32(s, pts, plan.pattern, (int)k, cfg, st);
                 else if (plan.path >= 1) e = launch_2d_tuned_f32(s, pts, plan.pattern, one, st);
                 else e = launch_2d_plain_f32(s, pts, bx, by, st);
+            }
+            if (plan.rtile && want_res && e == hipSuccess) {
+                e = launch_reduce_partials(g->d_partials, rtile2d_blocks((int)g->W, (int)g->H, rt), g->d_res + nr, st);
+                fused_res = true;
             }
         } else {
             Sweep3D s = make_sweep3d(g, src, dst, plan.radius, want_res ? g->d_partials : nullptr);
@@ -564,6 +579,22 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
 }  // namespace
 
 namespace {
+
+constexpr size_t kScratchPartials = 65536;  // partials of one launch (blocks) of an allocation-free run
+
+// the register tiles reach a field's rows through 32-bit buffer offsets
+bool cloud_fields_fit(const pskel_grid_t* g)
+{
+    for (int k = 0; k < 2; ++k) {
+        int fd;
+        size_t fw, fh, fz, fp;
+        const float* data;
+        if (!field_info(g->fields[k], &fd, &fw, &fh, &fz, &data, &fp) ||
+            (uint64_t)(g->H + 512) * fp * 4 >= 0x7fffffffull)
+            return false;
+    }
+    return true;
+}
 
 // Validate a run and choose its kernels (shared by the resident runner and the
 // host-staged pipeline).
@@ -639,6 +670,16 @@ pskel_status_t plan_run(const pskel_grid_t* g, const pskel_stencil_desc_t* d, co
                 if (radius != 1) return fail(PSKEL_ERR_UNSUPPORTED, "2D register march: mask range 1");
             }
         }
+        // fused sweeps of the radius-1 f32 stencils run on register tiles, whatever
+        // depth and tile the launch names
+        plan.rtile = tunable && ndim == 2 && g->storage == PSKEL_DTYPE_F32 && cfg.time_tile > 1 && radius == 1 &&
+                     rtile2d_ok(plan.pattern, (int)g->W, (int)g->H, g->pitch) &&
+                     (plan.pattern != PAT_CLOUD || cloud_fields_fit(g));
+        // the allocation-free run's partials hold 65536 blocks
+        if (plan.rtile && g->odd_2d_launches && cfg.residual_every > 0 &&
+            rtile2d_blocks((int)g->W, (int)g->H, rtile2d_plan(plan.pattern, (int)g->W, (int)g->H, 1, true)) >
+                kScratchPartials)
+            plan.rtile = false;
         if (cfg.time_tile > 3 && ndim == 3) return fail(PSKEL_ERR_UNSUPPORTED, "3D temporal depth above 3");
         // two or three fused sweeps per launch run the 7-point Jacobi; for any
         // other 3D stencil the depth is a hint and sweeps run singly
@@ -690,6 +731,9 @@ size_t residual_partials(const pskel_grid_t* g, const RunPlan& plan, const Point
                          const pskel_launch_cfg_t& cfg)
 {
     size_t nb = diff_blocks(g->nrows);
+    if (plan.rtile)
+        nb = std::max(nb, rtile2d_blocks((int)g->W, (int)g->H,
+                                         rtile2d_plan(plan.pattern, (int)g->W, (int)g->H, 1, g->odd_2d_launches)));
     if (g->ndim == 3 && plan.path == 3) {
         nb = std::max(nb, points3d_blocks(make_sweep3d(g, nullptr, nullptr, plan.radius, nullptr), pts));
     } else if (g->ndim == 3) {
@@ -721,7 +765,7 @@ pskel_status_t pskel::run_async(pskel_grid_t* g, const pskel_stencil_desc_t* d, 
     pskel_status_t st = plan_run(g, d, cfg, plan);
     if (st != PSKEL_OK) return st;
     if (iterations == 0) return PSKEL_OK;
-    if (plan.path == 2 && g->ndim == 2 && !g->buf[2]) return fail(PSKEL_ERR_RUNTIME, "spare buffer missing");
+    if ((plan.path == 2 || plan.rtile) && g->ndim == 2 && !g->buf[2]) return fail(PSKEL_ERR_RUNTIME, "spare buffer missing");
     Points pts;
     fill_points(pts, *d, g->ndim);
     int64_t nr = 0;
@@ -1030,7 +1074,7 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
         Sweep3D s3 = make_sweep3d(g, nullptr, nullptr, radius, nullptr);
         for (int k = 2; k <= std::max(2, cfg.time_tile); ++k) (void)ttile3d_blocks(s3, g->storage, cfg, k);
     }
-    if (plan.path == 2 && ndim == 2 && !g->buf[2]) {
+    if ((plan.path == 2 || plan.rtile) && ndim == 2 && !g->buf[2]) {
         PSKEL_HIP(hipMalloc(&g->buf[2], g->bytes));
         PSKEL_HIP(launch_copy(g->buf[2], g->buf[0], g->bytes, stream));
         g->spare_parity = g->parity;
@@ -1107,7 +1151,8 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
         // advance the host-side state exactly as the captured sequence did
         const int kmax = (plan.path == 2) ? std::max(1, cfg.time_tile) : 1;
         for (size_t done = 0; done < iterations;) {
-            const size_t k = next_k(done, iterations, kmax, every, g->ndim, g->odd_2d_launches);
+            RtPlan rt;
+            const size_t k = next_k(*g, plan, done, iterations, kmax, every, &rt);
             if (k % 2 == 0 && g->ndim == 2) g->spare_parity = g->parity;  // ring copy in the graph
             advance_state(*g, k);
             g->sweeps_done += k;
@@ -1141,7 +1186,6 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
 // not a device address on the host.
 // ---------------------------------------------------------------------------
 namespace {
-constexpr size_t kScratchPartials = 65536;   // partials of one launch (blocks)
 constexpr size_t kScratchResiduals = 4096;   // residuals of one call
 constexpr int kScratchDevices = 64;
 }  // namespace

@@ -200,6 +200,19 @@ hipError_t launch_2d_march_f32(const Sweep2D& s, const Points& p, int pattern, i
 // a grid the register march takes: wider than 8 cells, buffer under 2 GiB
 bool march2d_ok(int W, int H, size_t pitch);
 
+// Register tiles (k_rtile2d.hip): one launch's sweeps k and its tile (r rows per
+// wave, nw waves).
+struct RtPlan {
+    int r = 0, nw = 0, k = 0;
+};
+bool rtile2d_ok(int pattern, int W, int H, size_t pitch);
+// the next launch of a run with `rem` sweeps to go (odd: an odd number of them)
+RtPlan rtile2d_plan(int pattern, int W, int H, size_t rem, bool odd);
+size_t rtile2d_blocks(int W, int H, const RtPlan& q);
+// partials: with k = 1, one sum of squared changes per block
+hipError_t launch_2d_rtile(const Sweep2D& s, const Points& pts, const CloudArgs* cloud, int pattern, const RtPlan& q,
+                           double* partials, hipStream_t st);
+
 // arbitrary masks through an LDS tile (k_points.hip): masks whose halo fits it
 bool points2d_ok(int W, int H, const Points& p);
 hipError_t launch_2d_points_f32(const Sweep2D& s, const Points& p, hipStream_t st);
