@@ -109,9 +109,9 @@ typedef struct pskel_launch_cfg {
     int32_t tile_y;         /* tuned: rows per lane (2D) / w-rows per wave (3D) */
     int32_t tile_z;         /* tuned 3D: planes per block segment along h; 2D: waves per block */
     int32_t time_tile;      /* tuned: sweeps fused per launch (temporal depth k); 0/1 = none.
-                               2D f32 at mask range 1: any k > 1 (CLOUDSIM too) lets the run
-                               fuse as many sweeps per launch as pay on register tiles; the
-                               tiles below hold where those do not run (mask range above 1,
+                               2D at mask range 1: any k > 1 (CLOUDSIM and life too) lets the
+                               run fuse as many sweeps per launch as pay on register tiles;
+                               the tiles below hold where those do not run (mask range above 1,
                                grids up to 8 cells wide or over 2 GiB, the 9-point stencil
                                above 12M cells).
                                2D: k <= 4 (8 for life): tile (0, CY, 0) LDS tiles of CY in

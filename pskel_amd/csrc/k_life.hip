@@ -8,10 +8,11 @@
 //   k_life_swar   16 cells per lane packed in two u64 words; horizontal
 //                 neighbours by byte shifts plus one cross-lane exchange per row,
 //                 counts and rule evaluated bytewise (SWAR), RY rows per lane.
-//   k_life_bits   K generations per launch on
-//                 cells packed one bit each: each wave evolves its own tile
-//                 in registers.
+//   k_life_tiles  many generations per launch on cells packed one bit each, a
+//                 tile in the registers of a block (k_ltile.hpp).
 #include "k_tiles2d.hpp"
+#define PSKEL_LTILE_INSTANTIATE
+#include "k_ltile.hpp"
 
 namespace pskel {
 
@@ -45,45 +46,70 @@ __global__ __launch_bounds__(256) void k_life_swar(Sweep2D s)
     tile_life<RY>(s, blockIdx.x, blockIdx.y);
 }
 
-template <int K, int R>
-__global__ __launch_bounds__(256) void k_life_bits(Sweep2D s, int ntx, int ntiles)
-{
-    const int t = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-    if (t >= ntiles) return;  // whole waves; the tile body does not synchronise
-    life_bits_tile<K, R>(s, ntx, t, (int)threadIdx.x % kWave, K);
-}
-
 }  // namespace
 
-hipError_t launch_life_bits(const Sweep2D& s, int k, const pskel_launch_cfg_t& cfg, hipStream_t st)
+bool life_tiles_ok(size_t pitch) { return lt_fits(pitch); }
+
+static bool lt_depth_ok(int H, const RtPlan& q)
 {
-    // rows per lane: cfg.tile_y rounded up to 24, 32, 40, 48 or 64, and at
-    // least 2k + 8 (8 core rows)
-    int r = std::max(cfg.tile_y > 0 ? cfg.tile_y : 32, 2 * k + 8);
-    r = r <= 24 ? 24 : (r <= 32 ? 32 : (r <= 40 ? 40 : (r <= 48 ? 48 : 64)));
-    constexpr int CW = 62 * 32;
-    const int ntx = std::max(1, (s.W - 1 + CW - 1) / CW);
-#define PSKEL_LIFE_BITS(KV, RV)                                                                     \
-    if (k == KV && r == RV) {                                                                       \
-        const int nty = std::max(1, (s.H - 1 + (RV - 2 * KV) - 1) / (RV - 2 * KV));                 \
-        const int ntiles = ntx * nty;                                                               \
-        hipLaunchKernelGGL((k_life_bits<KV, RV>), dim3((ntiles + 3) / 4), dim3(256), 0, st, s, ntx, \
-                           ntiles);                                                                 \
-        return hipGetLastError();                                                                   \
-    }
-#define PSKEL_LIFE_BITS_K(KV)                                                                        \
-    PSKEL_LIFE_BITS(KV, 24) PSKEL_LIFE_BITS(KV, 32) PSKEL_LIFE_BITS(KV, 40) PSKEL_LIFE_BITS(KV, 48) \
-    PSKEL_LIFE_BITS(KV, 64)
-    PSKEL_LIFE_BITS_K(2)
-    PSKEL_LIFE_BITS_K(3)
-    PSKEL_LIFE_BITS_K(4)
-    PSKEL_LIFE_BITS_K(5)
-    PSKEL_LIFE_BITS_K(6)
-    PSKEL_LIFE_BITS_K(7)
-    PSKEL_LIFE_BITS_K(8)
-#undef PSKEL_LIFE_BITS_K
-#undef PSKEL_LIFE_BITS
-    return hipErrorInvalidValue;
+    return q.k >= 1 && q.k <= kLtMaxDepth && (H <= q.r * q.nw || 2 * q.k < q.r * q.nw);
+}
+
+// Tile shapes and the blocks of each that a CU holds, and the time of a launch in
+// microseconds: a launch, then rounds of blocks, each packing and unpacking its
+// rows and running its generations at the VALU's rate for the rows a CU holds
+// or, with few, at the latency of a barrier and one block's rows; no less than
+// its bytes take.  Fitted to 472 measured launches (64^2 to 8194^2, 1 to 30
+// generations): the fastest choice on all 8 boards.
+struct LtShape {
+    int r, nw, per_cu;
+};
+static constexpr LtShape kLtShapes[] = {{2, 8, 4}, {2, 16, 2}, {4, 16, 2}, {8, 8, 4}, {8, 16, 2}};
+
+static double lt_time(const LtShape& h, int W, int H, int k)
+{
+    constexpr double launch = 2.54, pack = 0.0442, row = 0.0093, barrier = 0.342, rate = 6.6e6;
+    constexpr int cus = 256;  // what the fit was measured on
+    const int rows = h.r * h.nw;
+    const int64_t nb = (int64_t)lt_tiles(W, kLtCols, 32) * lt_tiles(H, rows, k);
+    const int64_t slots = (int64_t)cus * h.per_cu, full = nb / slots, rest = nb % slots;
+    auto round = [&](int64_t b) {
+        return pack * (double)(b * rows) + k * std::max(row * (double)(b * rows), barrier + row * rows);
+    };
+    const double t = launch + (double)full * round(h.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0);
+    return std::max(t, launch + ((double)nb * kLtCols * rows + (double)W * H) / rate);
+}
+
+RtPlan life_tiles_plan(int W, int H, size_t rem, bool odd)
+{
+    return plan_fused(
+        kLtShapes, rem, odd, kLtMaxDepth,
+        [&](const LtShape& h, int k) {
+            RtPlan q;
+            q.r = h.r;
+            q.nw = h.nw;
+            q.k = k;
+            return lt_depth_ok(H, q);
+        },
+        [&](const LtShape& h, int k) { return lt_time(h, W, H, k); });
+}
+
+hipError_t launch_life_tiles(const Sweep2D& s, const RtPlan& q, hipStream_t st)
+{
+    if (!lt_fits(s.pitch) || !lt_depth_ok(s.H, q)) return hipErrorInvalidValue;
+    const int ntx = lt_tiles(s.W, kLtCols, 32);
+    const dim3 grid((unsigned)(ntx * lt_tiles(s.H, q.r * q.nw, q.k))), block(q.nw * kWave);
+#define PSKEL_LT(R, NW) \
+    if (q.r == R && q.nw == NW) hipLaunchKernelGGL((k_life_tiles<R, NW>), grid, block, 0, st, s, ntx, q.k)
+    // the shapes of kLtShapes
+    PSKEL_LT(2, 8);
+    else PSKEL_LT(2, 16);
+    else PSKEL_LT(4, 16);
+    else PSKEL_LT(8, 8);
+    else PSKEL_LT(8, 16);
+    else return hipErrorInvalidValue;
+#undef PSKEL_LT
+    return hipGetLastError();
 }
 
 hipError_t launch_life_plain(const Sweep2D& s, const Points& p, int bx, int by, hipStream_t st)

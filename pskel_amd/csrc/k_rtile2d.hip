@@ -67,32 +67,18 @@ double rt_time(const RtShape& h, int W, int H, int k)
 
 }  // namespace
 
-// The shape and depth with the least time for the run's remaining sweeps, cut
-// into launches of equal depth.  An even depth keeps the state's ring in place
-// (the next launch needs no ring copy); an odd one may end the run.
 RtPlan rtile2d_plan(int pattern, int W, int H, size_t rem, bool odd)
 {
-    RtPlan best;
-    double best_t = 0.0;
-    for (const RtShape& h : kRtShapes) {
-        if (h.pattern != pattern) continue;
-        for (int k = 1; k <= kRtMaxDepth && (size_t)k <= rem; ++k) {
-            const RtPlan q{h.r, h.nw, k};
-            if (!rt_depth_ok(W, H, q)) break;
-            if ((size_t)k != rem && k != 1 && (k % 2 == 1) != odd) continue;
-            if (odd && k % 2 == 0) continue;
-            const double t = rt_time(h, W, H, k) * (double)((rem + k - 1) / k);
-            if (best.k && t >= best_t) continue;
-            best = q;
-            best_t = t;
-        }
-    }
-    // the same number of launches, evened out
-    const size_t n = (rem + best.k - 1) / best.k;
-    size_t k = (rem + n - 1) / n;
-    if (n > 1 && (k % 2 == 1) != odd) k += 1;
-    best.k = (int)std::min<size_t>(k, (size_t)best.k);
-    return best;
+    return plan_fused(
+        kRtShapes, rem, odd, kRtMaxDepth,
+        [&](const RtShape& h, int k) {
+            RtPlan q;
+            q.r = h.r;
+            q.nw = h.nw;
+            q.k = k;
+            return h.pattern == pattern && rt_depth_ok(W, H, q);
+        },
+        [&](const RtShape& h, int k) { return rt_time(h, W, H, k); });
 }
 
 namespace {

@@ -429,7 +429,8 @@ size_t next_k(const pskel::Grid& g, const RunPlan& plan, size_t done, size_t ite
         if (g.ndim == 2 && k > 1 && (done + k) % every == 0) k -= 1;
     }
     if (plan.rtile) {
-        *rt = rtile2d_plan(plan.pattern, (int)g.W, (int)g.H, k, g.odd_2d_launches);
+        *rt = plan.pattern == PAT_LIFE8 ? life_tiles_plan((int)g.W, (int)g.H, k, g.odd_2d_launches)
+                                        : rtile2d_plan(plan.pattern, (int)g.W, (int)g.H, k, g.odd_2d_launches);
         return (size_t)rt->k;
     }
     if (g.odd_2d_launches && g.ndim == 2 && k % 2 == 0) k -= 1;
@@ -512,7 +513,7 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
                 else if (plan.path >= 1) e = launch_cloud_tuned(s, ca, one, st);
                 else e = launch_cloud_plain(s, ca, bx, by, st);
             } else if (g->storage == PSKEL_DTYPE_U8) {
-                if (k > 1) e = launch_life_bits(s, (int)k, cfg, st);
+                if (plan.rtile && !want_res) e = launch_life_tiles(s, rt, st);
                 else if (plan.path >= 1) e = launch_life_tuned(s, one, st);
                 else e = launch_life_plain(s, pts, bx, by, st);
             } else {
@@ -525,7 +526,7 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
                 else if (plan.path >= 1) e = launch_2d_tuned_f32(s, pts, plan.pattern, one, st);
                 else e = launch_2d_plain_f32(s, pts, bx, by, st);
             }
-            if (plan.rtile && want_res && e == hipSuccess) {
+            if (plan.rtile && plan.pattern != PAT_LIFE8 && want_res && e == hipSuccess) {
                 e = launch_reduce_partials(g->d_partials, rtile2d_blocks((int)g->W, (int)g->H, rt), g->d_res + nr, st);
                 fused_res = true;
             }
@@ -672,11 +673,13 @@ pskel_status_t plan_run(const pskel_grid_t* g, const pskel_stencil_desc_t* d, co
         }
         // fused sweeps of the radius-1 f32 stencils run on register tiles, whatever
         // depth and tile the launch names
-        plan.rtile = tunable && ndim == 2 && g->storage == PSKEL_DTYPE_F32 && cfg.time_tile > 1 && radius == 1 &&
+        if (plan.pattern == PAT_LIFE8 && plan.path == 2 && !life_tiles_ok(g->pitch)) plan.path = 1;
+        if (plan.pattern == PAT_LIFE8 && plan.path == 2) plan.rtile = true;
+        else plan.rtile = tunable && ndim == 2 && g->storage == PSKEL_DTYPE_F32 && cfg.time_tile > 1 && radius == 1 &&
                      rtile2d_ok(plan.pattern, (int)g->W, (int)g->H, g->pitch) &&
                      (plan.pattern != PAT_CLOUD || cloud_fields_fit(g));
         // the allocation-free run's partials hold 65536 blocks
-        if (plan.rtile && g->odd_2d_launches && cfg.residual_every > 0 &&
+        if (plan.rtile && plan.pattern != PAT_LIFE8 && g->odd_2d_launches && cfg.residual_every > 0 &&
             rtile2d_blocks((int)g->W, (int)g->H, rtile2d_plan(plan.pattern, (int)g->W, (int)g->H, 1, true)) >
                 kScratchPartials)
             plan.rtile = false;
@@ -731,7 +734,7 @@ size_t residual_partials(const pskel_grid_t* g, const RunPlan& plan, const Point
                          const pskel_launch_cfg_t& cfg)
 {
     size_t nb = diff_blocks(g->nrows);
-    if (plan.rtile)
+    if (plan.rtile && plan.pattern != PAT_LIFE8)
         nb = std::max(nb, rtile2d_blocks((int)g->W, (int)g->H,
                                          rtile2d_plan(plan.pattern, (int)g->W, (int)g->H, 1, g->odd_2d_launches)));
     if (g->ndim == 3 && plan.path == 3) {

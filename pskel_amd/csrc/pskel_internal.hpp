@@ -205,6 +205,37 @@ bool march2d_ok(int W, int H, size_t pitch);
 struct RtPlan {
     int r = 0, nw = 0, k = 0;
 };
+// The shape and depth with the least time for the run's remaining `rem` sweeps,
+// cut into launches of equal depth.  An even depth keeps the state's ring in
+// place (the next launch needs no ring copy); an odd one may end the run, and
+// is all there is without a spare buffer (odd).  Shape: {r, nw, ...}; ok(shape,
+// k): the tile is deep enough; time(shape, k): of one launch.
+template <class Shape, size_t N, class Ok, class Time>
+RtPlan plan_fused(const Shape (&shapes)[N], size_t rem, bool odd, int kmax, Ok ok, Time time)
+{
+    RtPlan best;
+    double best_t = 0.0;
+    for (const Shape& h : shapes) {
+        for (int k = 1; k <= kmax && (size_t)k <= rem; ++k) {
+            if (!ok(h, k)) break;
+            if ((size_t)k != rem && k != 1 && (k % 2 == 1) != odd) continue;
+            if (odd && k % 2 == 0) continue;
+            const double t = time(h, k) * (double)((rem + k - 1) / k);
+            if (best.k && t >= best_t) continue;
+            best.r = h.r;
+            best.nw = h.nw;
+            best.k = k;
+            best_t = t;
+        }
+    }
+    // the same number of launches, evened out
+    const size_t n = (rem + best.k - 1) / best.k;
+    size_t k = (rem + n - 1) / n;
+    if (n > 1 && (k % 2 == 1) != odd) k += 1;
+    best.k = (int)std::min<size_t>(k, (size_t)best.k);
+    return best;
+}
+
 bool rtile2d_ok(int pattern, int W, int H, size_t pitch);
 // the next launch of a run with `rem` sweeps to go (odd: an odd number of them)
 RtPlan rtile2d_plan(int pattern, int W, int H, size_t rem, bool odd);
@@ -222,7 +253,10 @@ size_t points3d_blocks(const Sweep3D& s, const Points& p);  // 0: the halo does 
 // 2D life (u8) sweeps.
 hipError_t launch_life_plain(const Sweep2D& s, const Points& p, int bx, int by, hipStream_t st);
 hipError_t launch_life_tuned(const Sweep2D& s, const pskel_launch_cfg_t& cfg, hipStream_t st);
-hipError_t launch_life_bits(const Sweep2D& s, int k, const pskel_launch_cfg_t& cfg, hipStream_t st);
+// bit-packed tiles (k_ltile.hpp), plan and launch as the register tiles above
+bool life_tiles_ok(size_t pitch);
+RtPlan life_tiles_plan(int W, int H, size_t rem, bool odd);
+hipError_t launch_life_tiles(const Sweep2D& s, const RtPlan& q, hipStream_t st);
 
 // 3D sweeps for every storage type.
 hipError_t launch_3d_plain(const Sweep3D& s, const Points& p, int storage, int bx, int by,
