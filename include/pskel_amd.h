@@ -343,17 +343,17 @@ pskel_status_t pskel_grid_set_field(pskel_grid_t* grid, int32_t slot, pskel_fiel
  *      reference runs one Stencil at a time with a launch and a host sync per
  *      sweep (include/PSkelStencil.hpp:1078-1082, 1790-1791).
  *      Grids: 2D, one device, Jacobi 5-point or 3x3 weighted (F32) or life
- *      (U8).  cfgs[i].time_tile is grid i's temporal depth, the sweeps it fuses
- *      per launch: 1 (or 0) or 3 for F32 (LDS temporal tiles), 1, 3, 5 or 7
- *      for life (bit-packed tiles, mask range 1); odd, so every launch moves a
- *      grid's state to its other buffer.  N sweeps run as N / k launches of k
- *      and the rest as one odd launch or two (r - 1, then 1).  cfgs[i].tile_y:
- *      at depth 1 the rows per lane (1, 2, 4, 8; default 4), at depth 3 in F32
- *      the tile rows (16 or 32; default 16).  F32 at depth 3 with tile_x = 4
- *      runs the register march instead (mask range 1, grids over 8 cells wide):
- *      one wave per tile of 62 x 4 columns and segment of tile_z rows (0: 32),
- *      its single-sweep tail launches through register tiles.  cfgs may be
- *      NULL (depth 1, 4 rows). */
+ *      (U8).  cfgs[i].time_tile is grid i's temporal depth, the least sweeps it
+ *      fuses per launch: 1 (or 0) or 3 for F32, 1, 3, 5 or 7 for life (mask
+ *      range 1).  Above 1, life and F32 at mask range 1 run on tiles held in
+ *      registers, at the depth that suits the batch and the run's length; F32
+ *      at a wider range runs LDS tiles of tile_y rows (16 or 32; default 16).
+ *      A launch fuses an odd number k, so it moves a grid's state to its other
+ *      buffer: N sweeps run as N / k launches of k and the rest as one odd
+ *      launch or two (r - 1, then 1).  At depth 1 cfgs[i].tile_y is the rows
+ *      per lane (1, 2, 4, 8; default 4).  tile_x = 4 at depth 3 (the register
+ *      march's launch) is accepted for grids over 8 cells wide and runs the
+ *      same register tiles.  cfgs may be NULL (depth 1, 4 rows). */
 typedef struct pskel_batch pskel_batch_t;
 pskel_status_t pskel_batch_create(pskel_grid_t* const* grids, const pskel_stencil_desc_t* descs,
                                   const pskel_launch_cfg_t* cfgs, size_t n, pskel_batch_t** out);

@@ -207,13 +207,13 @@ class Field:
 
 
 class Batch:
-    """Many 2D grids swept together by one persistent kernel per launch
-    (pskel_batch_t).  grids: list of Grid; stencils: one per grid; rows: rows
-    per lane per grid (1, 2, 4 or 8) at depth 1, tile rows at depth > 1 (f32:
-    16 or 32; life: 32); depths: sweeps fused per launch per grid (odd: 1 or 3
-    for f32, 1, 3, 5 or 7 for life); march: per grid, 0 or, for an f32 grid at
-    depth 3, the rows per segment of the register march that replaces its LDS
-    tiles (tile (4, 0, rows))."""
+    """Many 2D grids swept together by persistent kernels (pskel_batch_t).
+    grids: list of Grid; stencils: one per grid; depths: least sweeps fused per
+    launch per grid (odd: 1 or 3 for f32, 1, 3, 5 or 7 for life); rows: rows per
+    lane per grid (1, 2, 4 or 8) at depth 1, rows of the LDS tiles (16 or 32)
+    where an f32 grid at depth 3 runs those (a mask range above 1); march: per
+    grid, 0 or, for an f32 grid at depth 3, a register march's rows per segment
+    (the same register tiles run either way)."""
 
     def __init__(self, grids, stencils, rows=None, depths=None, march=None):
         n = len(grids)

@@ -12,8 +12,12 @@
 // with the other families' (no grid belongs to two).
 //
 // Temporal depth.  Each grid fuses K sweeps per launch (K odd: 1 or 3 for the
-// f32 stencils, through the LDS temporal tile; 1, 3, 5 or 7 for life, through
-// the bit-packed tile; K = 1 runs the register tiles).  An odd number of sweeps
+// f32 stencils, on register tiles (k_rtile2d.hpp) or, where those do not run,
+// the LDS temporal tile; 1, 3, 5 or 7 for life, on bit-packed tiles
+// (k_ltile.hpp); K = 1 runs the one-sweep tiles of k_tiles2d.hpp).  A grid of
+// a family that holds its tiles in registers (bit-packed life, the f32 register
+// tiles) fuses as many sweeps as pay for the whole family, at least the depth
+// asked for: plan_batch picks it for each run length.  An odd number of sweeps
 // per launch moves the state to the other buffer, so grid g's launch l reads
 // buffer l & 1 and writes the other, with no third buffer.  N sweeps of grid g
 // run as N / K launches of K, then the rest r = N mod K as one launch of r
@@ -25,8 +29,11 @@
 #include <vector>
 
 #include "k_tiles2d.hpp"
-#define PSKEL_MARCH2D_INSTANTIATE
 #include "k_march2d.hpp"
+#define PSKEL_RTILE_INSTANTIATE
+#include "k_rtile2d.hpp"
+#define PSKEL_LTILE_INSTANTIATE
+#include "k_ltile.hpp"
 
 using namespace pskel;
 
@@ -41,10 +48,9 @@ struct BatchEntry {
     int pitch;
     int radius;
     int kind;
-    int ry;           // K = 1: rows per lane; K > 1: tile rows (f32: CY; life: bit-tile rows R;
-                      // register march: rows per segment)
-    int march;        // f32 at K = 3 through the register march (one wave per tile and segment)
-    int depth;        // K, sweeps fused per launch (odd)
+    int ry;           // K = 1: rows per lane; LDS tiles: tile rows
+    int rtile;        // f32 at K = 3 on register tiles
+    int depth;        // K, sweeps fused per launch (odd); of a tile family: the tiles' halo
     int full;         // launches of K sweeps
     int tail0, tail1; // sweeps of the launches after them (odd; 0: none)
     int tiles_x;      // tiles along w
@@ -57,7 +63,11 @@ struct BatchEntry {
 constexpr int kBatchWaves = 4;  // block = (64, 4)
 constexpr int kTTileCX = 120;   // columns of an f32 temporal tile
 constexpr int kTTileK = 3;      // depth of the f32 temporal tiles
-constexpr int kLifeRows = 32;   // rows of a bit-packed life tile
+// register and bit-packed life tiles: 8 waves of 8 rows (a 64-row tile keeps 58
+// rows of its own at 3 sweeps, 50 at 7 generations)
+constexpr int kBatchTileWaves = 8;
+constexpr int kBatchTileRows = 8;
+constexpr int kBatchTileH = kBatchTileWaves * kBatchTileRows;
 constexpr int kBatchLds = ttile_lds<kTTileK, kTTileCX, 32>();  // floats per LDS buffer (the largest tile)
 
 __device__ __forceinline__ int sweeps_of(const BatchEntry& E, int launch)
@@ -90,51 +100,31 @@ __device__ __forceinline__ void run_ttile(const BatchEntry& E, const Sweep2D& s,
     else ttile_body<PAT, kTTileK, kTTileCX, 32>(s, E, tx, ty, k, tid, A, B);
 }
 
-__device__ __forceinline__ void run_life_bits(const BatchEntry& E, const Sweep2D& s, int item_t, int k)
-{
-    // an item is four bit tiles, one per wave
-    const int t = item_t * kBatchWaves + (int)threadIdx.y;
-    if (t >= E.ntiles) return;  // a whole wave; the tile body does not synchronise
-    const int lane = (int)threadIdx.x;
-    switch (E.depth) {
-    case 3: life_bits_tile<3, kLifeRows>(s, E.tiles_x, t, lane, k); break;
-    case 5: life_bits_tile<5, kLifeRows>(s, E.tiles_x, t, lane, k); break;
-    default: life_bits_tile<7, kLifeRows>(s, E.tiles_x, t, lane, k); break;
-    }
-}
-
-// A register-march grid: launches of 3 sweeps run one wave per (tile,
-// segment) unit, four units per item; its single-sweep tail launches cover the
-// grid with register tiles of 4 rows per lane (256 columns x 16 rows), each
-// of the grid's items taking every items-th tile.
-__device__ __forceinline__ void run_march(const BatchEntry& E, const Sweep2D& s, int item_t, int k)
-{
-    const int lane = (int)threadIdx.x, wave = (int)threadIdx.y;
-    if (k == 3) {
-        const int g = item_t * kBatchWaves + wave;
-        if (g >= E.ntiles) return;  // the whole wave; the march does not synchronise
-        if (E.kind == BK_J5) march2d_wave<PAT_J5, 3, 3>(s, E, E.tiles_x, E.ry, g, lane);
-        else march2d_wave<PAT_BOX9, 3, 3>(s, E, E.tiles_x, E.ry, g, lane);
-        return;
-    }
-    const int ni = (E.ntiles + kBatchWaves - 1) / kBatchWaves;  // the grid's items
-    const int rtx = (E.W + 255) / 256, nrt = rtx * ((E.H + 4 * kBatchWaves - 1) / (4 * kBatchWaves));
-    for (int rt = item_t; rt < nrt; rt += ni) {
-        if (E.kind == BK_J5) tile_f32<PAT_J5, 4>(s, E, rt % rtx, rt / rtx);
-        else tile_f32<PAT_BOX9, 4>(s, E, rt % rtx, rt / rtx);
-    }
-}
-
 // Work families, one kernel each so each keeps the registers its body needs
-// (register and SWAR tiles, f32 LDS temporal tiles, bit-packed life tiles,
-// register-march units).
-enum BatchFamily : int { BF_REG = 0, BF_TTILE = 1, BF_BITS = 2, BF_MARCH = 3, BF_COUNT = 4 };
+// (one-sweep tiles, f32 LDS temporal tiles, bit-packed life tiles, f32 register
+// tiles of the 5-point and the 3x3 stencil, which need 79 and 91 registers, and
+// 130 in one kernel).
+enum BatchFamily : int { BF_REG = 0, BF_TTILE = 1, BF_BITS = 2, BF_J5 = 3, BF_BOX9 = 4, BF_COUNT = 5 };
+
+// waves per block
+constexpr int fam_waves(int fam) { return fam >= BF_BITS ? kBatchTileWaves : kBatchWaves; }
 
 template <int FAM>
-__global__ __launch_bounds__(256) void k_batch(const BatchEntry* __restrict__ tab, const int* __restrict__ item_grid,
+struct FamLds {
+    float lds[FAM == BF_TTILE ? 2 * kBatchLds : 1];
+};
+template <>
+struct FamLds<BF_BITS> : LtLds<kBatchTileRows, kBatchTileWaves> {};
+template <>
+struct FamLds<BF_J5> : RtLds<kBatchTileRows, kBatchTileWaves> {};
+template <>
+struct FamLds<BF_BOX9> : RtLds<kBatchTileRows, kBatchTileWaves> {};
+
+template <int FAM>
+__global__ __launch_bounds__(fam_waves(FAM) * kWave) void k_batch(const BatchEntry* __restrict__ tab, const int* __restrict__ item_grid,
                                                int nitems, int launch)
 {
-    __shared__ float lds[FAM == BF_TTILE ? 2 * kBatchLds : 1];
+    __shared__ FamLds<FAM> L;
     const int parity = launch & 1;
     for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
         const int g = item_grid[item];
@@ -157,13 +147,23 @@ __global__ __launch_bounds__(256) void k_batch(const BatchEntry* __restrict__ ta
             case 4: run_item<4>(E, s, t); break;
             default: run_item<8>(E, s, t); break;
             }
-        } else if constexpr (FAM == BF_BITS) {
-            run_life_bits(E, s, t, k);
-        } else if constexpr (FAM == BF_MARCH) {
-            run_march(E, s, t, k);
+        } else if constexpr (FAM >= BF_BITS) {
+            const int lane = (int)threadIdx.x, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+            const int tx = t % E.tiles_x, ty = t / E.tiles_x;
+            if constexpr (FAM == BF_BITS) {
+                life_tile(s, tx, ty, E.depth, k, lane, wave, L);
+            } else {
+                RtParams p;
+                p.coeff = E.coeff;
+#pragma unroll
+                for (int i = 0; i < 9; ++i) p.wt[i] = E.wt[i];
+                rt_tile<FAM == BF_J5 ? PAT_J5 : PAT_BOX9, kBatchTileRows, kBatchTileWaves, false>(s, p, tx, ty, E.depth, k,
+                                                                                                 lane, wave, L);
+            }
+            __syncthreads();  // the next item's first rows go where this one's last may still be read
         } else {
-            if (E.kind == BK_J5) run_ttile<PAT_J5>(E, s, t, k, lds, lds + kBatchLds);
-            else run_ttile<PAT_BOX9>(E, s, t, k, lds, lds + kBatchLds);
+            if (E.kind == BK_J5) run_ttile<PAT_J5>(E, s, t, k, L.lds, L.lds + kBatchLds);
+            else run_ttile<PAT_BOX9>(E, s, t, k, L.lds, L.lds + kBatchLds);
         }
     }
 }
@@ -172,7 +172,8 @@ int family_of(const BatchEntry& e)
 {
     if (e.depth == 1) return BF_REG;
     if (e.kind == BK_LIFE) return BF_BITS;
-    return e.march ? BF_MARCH : BF_TTILE;
+    if (e.rtile) return e.kind == BK_J5 ? BF_J5 : BF_BOX9;
+    return BF_TTILE;
 }
 
 // the schedule of N sweeps at depth K: full launches of K, then the tail
@@ -189,15 +190,19 @@ void schedule(BatchEntry& e, size_t n)
     }
 }
 
-int launches_of(const BatchEntry& e) { return e.full + (e.tail0 > 0) + (e.tail1 > 0); }
-
-// items of one grid: register and SWAR tiles and f32 temporal tiles are one
-// block each, bit-packed life tiles and register-march units one wave each
-// (four per item)
-int items_of(const BatchEntry& e)
+// tiles of a grid of a register-tile family at depth K
+void tile_grid(BatchEntry& e, int K)
 {
-    return (e.kind == BK_LIFE && e.depth > 1) || e.march ? (e.ntiles + kBatchWaves - 1) / kBatchWaves : e.ntiles;
+    e.depth = K;
+    if (e.kind == BK_LIFE) {
+        e.tiles_x = lt_tiles(e.W, kLtCols, 32);
+    } else {
+        e.tiles_x = rt_tiles(e.W, kRtCols, rt_halo_cols(K));
+    }
+    e.ntiles = e.tiles_x * rt_tiles(e.H, kBatchTileH, K);
 }
+
+int launches_of(const BatchEntry& e) { return e.full + (e.tail0 > 0) + (e.tail1 > 0); }
 
 }  // namespace
 
@@ -206,6 +211,9 @@ struct pskel_batch {
     std::vector<BatchEntry> host_tab;
     BatchEntry* d_tab = nullptr;
     int* d_items = nullptr;          // the work items of each family, one list after the other
+    size_t items_cap = 0;
+    std::vector<int> asked;          // depth asked for each grid
+    int fam_slots[BF_COUNT] = {};    // blocks of a family's kernel the device holds at once
     int fam_items[BF_COUNT] = {};    // items per family
     int fam_first[BF_COUNT] = {};    // offset of a family's list in d_items
     int fam_blocks[BF_COUNT] = {};   // persistent blocks of a family's kernel
@@ -228,11 +236,89 @@ struct pskel_batch {
 
 namespace {
 
-// Schedules and item order for `n` sweeps: in each family's list, grids with
-// more launches first.
+// items per family, their places in the list, and the blocks that walk them: at
+// most as many as the device holds at once, so no block waits for a slot with a
+// full share of items
+void count_items(pskel_batch_t* b)
+{
+    b->nitems = 0;
+    for (int f = 0; f < BF_COUNT; ++f) b->fam_items[f] = 0;
+    for (const auto& e : b->host_tab) {
+        b->fam_items[family_of(e)] += e.ntiles;
+        b->nitems += e.ntiles;
+    }
+    for (int f = 0; f < BF_COUNT; ++f) {
+        b->fam_first[f] = f ? b->fam_first[f - 1] + b->fam_items[f - 1] : 0;
+        b->fam_blocks[f] = std::max(1, std::min(b->fam_items[f], b->fam_slots[f]));
+    }
+}
+
+// The depth of a register-tile family for runs of n sweeps: odd, at least the
+// least one asked for and at most n, with the least time for the run's launches
+// (the tiles' halo grows with it, the crossings of memory and the launches get
+// fewer).  A batched launch costs about 8 us more than one of a single grid (the
+// item and table lookups, the graph's steps).  Measured, 105 sweeps of the f32
+// half of 16, 48 and 256 grids of 64 to 2048 a side: depth 3 285, 573 and 2061
+// us; the picks 21, 13 and 7 185, 332 and 1270; the life half: depth 7 216, 287
+// and 600 us; the picks 21, 15 and 7 168, 238 and 600.
+constexpr double kBatchLaunchUs = 8.0;
+
+int family_depth(const pskel_batch_t* b, int f, size_t n)
+{
+    const bool life = f == BF_BITS;
+    int lo = 0;
+    double cells = 0.0;
+    for (size_t i = 0; i < b->host_tab.size(); ++i) {
+        const BatchEntry& e = b->host_tab[i];
+        if (family_of(e) != f) continue;
+        lo = lo ? std::min(lo, b->asked[i]) : b->asked[i];
+        cells += (double)e.W * e.H;
+    }
+    int best = lo;
+    double best_t = 0.0;
+    for (int K = lo; K <= 21 && (K == lo || (size_t)K <= n); K += 2) {
+        int64_t nb = 0;
+        for (const BatchEntry& e : b->host_tab) {
+            if (family_of(e) != f) continue;
+            BatchEntry t = e;
+            tile_grid(t, K);
+            nb += t.ntiles;
+        }
+        BatchEntry t{};
+        t.depth = K;
+        schedule(t, n);
+        const int per_cu = std::max(1, b->fam_slots[f] / kRtCus);
+        const double one = life ? lt_launch_time(kBatchTileH, per_cu, nb, cells, K)
+                                : rt_launch_time(f == BF_J5 ? PAT_J5 : PAT_BOX9, kBatchTileH, per_cu, nb, cells, K);
+        const double time = (one + kBatchLaunchUs) * launches_of(t);
+        if (K == lo || time < best_t) {
+            best = K;
+            best_t = time;
+        }
+    }
+    return best;
+}
+
+// Depths, schedules and item order for `n` sweeps: in each family's list, grids
+// with more launches first.
 pskel_status_t plan_batch(pskel_batch_t* b, size_t n)
 {
     const size_t ng = b->host_tab.size();
+    for (int f = BF_BITS; f < BF_COUNT; ++f) {
+        if (b->fam_items[f] == 0) continue;
+        const int K = family_depth(b, f, n);
+        for (auto& e : b->host_tab)
+            if (family_of(e) == f) tile_grid(e, K);
+    }
+    count_items(b);
+    if ((size_t)b->nitems > b->items_cap) {
+        // the list of the last run length is no longer in use: runs wait for their launches
+        if (b->d_items) (void)hipFree(b->d_items);
+        b->d_items = nullptr;
+        b->items_cap = 0;
+        PSKEL_HIP(hipMalloc(&b->d_items, (size_t)b->nitems * sizeof(int)));
+        b->items_cap = (size_t)b->nitems;
+    }
     for (auto& e : b->host_tab) schedule(e, n);
     std::vector<int> order(ng);
     std::iota(order.begin(), order.end(), 0);
@@ -250,7 +336,7 @@ pskel_status_t plan_batch(pskel_batch_t* b, size_t n)
         BatchEntry& e = b->host_tab[g];
         const int f = family_of(e);
         e.item0 = fill[f];
-        const int ni = items_of(e);
+        const int ni = e.ntiles;
         for (int t = 0; t < ni; ++t) items[(size_t)(b->fam_first[f] + fill[f]++)] = g;
         for (int l = 0; l < launches_of(e); ++l) b->launch_items[f][l] += ni;
     }
@@ -278,7 +364,6 @@ pskel_status_t refresh_table(pskel_batch_t* b)
 // and joined back into it (under capture: parallel branches of the graph).
 hipError_t issue_batch(pskel_batch_t* b, hipStream_t st)
 {
-    const dim3 block(kWave, kBatchWaves);
     hipError_t e = hipEventRecord(b->fork, st);
     for (int f = 0; f < BF_COUNT && e == hipSuccess; ++f) {
         if (b->fam_items[f] == 0) continue;
@@ -288,11 +373,12 @@ hipError_t issue_batch(pskel_batch_t* b, hipStream_t st)
         for (int l = 0; l < b->nlaunch && e == hipSuccess; ++l) {
             const int n = b->launch_items[f][l];
             if (n == 0) continue;
-            const dim3 grid((unsigned)std::min(n, b->fam_blocks[f]));
+            const dim3 grid((unsigned)std::min(n, b->fam_blocks[f])), block(kWave, fam_waves(f));
             if (f == BF_REG) hipLaunchKernelGGL(k_batch<BF_REG>, grid, block, 0, fs, b->d_tab, items, n, l);
             else if (f == BF_TTILE) hipLaunchKernelGGL(k_batch<BF_TTILE>, grid, block, 0, fs, b->d_tab, items, n, l);
             else if (f == BF_BITS) hipLaunchKernelGGL(k_batch<BF_BITS>, grid, block, 0, fs, b->d_tab, items, n, l);
-            else hipLaunchKernelGGL(k_batch<BF_MARCH>, grid, block, 0, fs, b->d_tab, items, n, l);
+            else if (f == BF_J5) hipLaunchKernelGGL(k_batch<BF_J5>, grid, block, 0, fs, b->d_tab, items, n, l);
+            else hipLaunchKernelGGL(k_batch<BF_BOX9>, grid, block, 0, fs, b->d_tab, items, n, l);
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = hipEventRecord(b->join[f], fs);
@@ -314,7 +400,6 @@ pskel_status_t pskel_batch_create(pskel_grid_t* const* grids, const pskel_stenci
         if (!grids[i]) return fail(PSKEL_ERR_INVALID_ARGUMENT, "batch grid is NULL");
     auto* b = new pskel_batch_t();
     b->device = grids[0]->device;
-    int nitems = 0;
     for (size_t i = 0; i < n; ++i) {
         pskel_grid_t* g = grids[i];
         auto reject = [&](pskel_status_t st, const char* msg) {
@@ -348,59 +433,61 @@ pskel_status_t pskel_batch_create(pskel_grid_t* const* grids, const pskel_stenci
             e.tiles_x = (e.W + cols - 1) / cols;
             e.ntiles = e.tiles_x * ((e.H + kBatchWaves * ry - 1) / (kBatchWaves * ry));
         } else if (e.kind == BK_LIFE) {
-            // bit-packed tiles of 32 rows, 3, 5 or 7 generations per launch
+            // bit-packed tiles, 3, 5 or 7 generations per launch
             if (depth != 3 && depth != 5 && depth != 7)
                 return reject(PSKEL_ERR_UNSUPPORTED, "batched life depths are 1, 3, 5 or 7");
             if (radius != 1) return reject(PSKEL_ERR_UNSUPPORTED, "batched life temporal tiles need mask range 1");
-            e.ry = kLifeRows;
-            constexpr int CW = 62 * 32;
-            const int cr = kLifeRows - 2 * depth;
-            e.tiles_x = std::max(1, (e.W - 1 + CW - 1) / CW);
-            e.ntiles = e.tiles_x * std::max(1, (e.H - 1 + cr - 1) / cr);
-        } else if (cfgs && cfgs[i].tile_x == kMarch2DVd) {
-            // register march, 3 sweeps per launch: tiles of 62 lane vectors along w,
-            // segments of tile_z rows (0: 32)
-            if (depth != 3) return reject(PSKEL_ERR_UNSUPPORTED, "the batched register march runs 3 sweeps per launch");
-            if (radius != 1 || !march2d_fits(e.W, e.H, g->pitch))
-                return reject(PSKEL_ERR_UNSUPPORTED, "the batched register march needs mask range 1 and a grid over 8 cells wide");
-            const March2DShape m = march2d_shape(e.W, e.H, cfgs[i].tile_z > 0 ? cfgs[i].tile_z : 32);
-            if (m.units < 1) return reject(PSKEL_ERR_UNSUPPORTED, "the batched register march needs interior rows");
-            e.march = 1;
-            e.ry = m.seg;
-            e.tiles_x = m.ntw;
-            e.ntiles = m.units;
+            if (lt_fits(g->pitch)) {
+                tile_grid(e, depth);
+            } else {  // boards of 8M columns: a generation per launch
+                e.depth = 1;
+                e.ry = 4;
+                e.tiles_x = (e.W + 1023) / 1024;
+                e.ntiles = e.tiles_x * ((e.H + kBatchWaves * 4 - 1) / (kBatchWaves * 4));
+            }
         } else {
-            // LDS temporal tiles of 120 columns and 16 or 32 rows, 3 sweeps per launch
+            // 3 sweeps per launch: the register tiles, whatever tile the launch
+            // names; LDS tiles of 120 columns and 16 or 32 rows at a mask range
+            // above 1 and on grids the register tiles do not take
+            const bool march = cfgs && cfgs[i].tile_x == kMarch2DVd;
+            if (march) {
+                if (depth != 3) return reject(PSKEL_ERR_UNSUPPORTED, "the batched register march runs 3 sweeps per launch");
+                if (radius != 1 || !march2d_fits(e.W, e.H, g->pitch))
+                    return reject(PSKEL_ERR_UNSUPPORTED, "the batched register march needs mask range 1 and a grid over 8 cells wide");
+                if (march2d_shape(e.W, e.H, 0).units < 1)
+                    return reject(PSKEL_ERR_UNSUPPORTED, "the batched register march needs interior rows");
+            }
             if (depth != kTTileK) return reject(PSKEL_ERR_UNSUPPORTED, "batched f32 depths are 1 or 3");
-            const int cy = cfgs && cfgs[i].tile_y > 0 ? cfgs[i].tile_y : 16;
+            const int cy = cfgs && cfgs[i].tile_y > 0 && !march ? cfgs[i].tile_y : 16;
             if (cy != 16 && cy != 32) return reject(PSKEL_ERR_UNSUPPORTED, "batched f32 temporal tiles have 16 or 32 rows");
-            e.ry = cy;
-            e.tiles_x = (e.W + kTTileCX - 1) / kTTileCX;
-            e.ntiles = e.tiles_x * ((e.H + cy - 1) / cy);
+            if (radius == 1 && rt_fits(e.W, e.H, g->pitch)) {
+                e.rtile = 1;
+                tile_grid(e, depth);
+            } else {
+                e.ry = cy;
+                e.tiles_x = (e.W + kTTileCX - 1) / kTTileCX;
+                e.ntiles = e.tiles_x * ((e.H + cy - 1) / cy);
+            }
         }
-        nitems += items_of(e);
-        b->fam_items[family_of(e)] += items_of(e);
         b->grids.push_back(g);
         b->host_tab.push_back(e);
+        b->asked.push_back(depth);
     }
-    b->nitems = nitems;
-    for (int f = 1; f < BF_COUNT; ++f) b->fam_first[f] = b->fam_first[f - 1] + b->fam_items[f - 1];
     hipError_t e = hipSetDevice(b->device);
     int cus = 256;
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device);
-    // persistent: at most as many blocks as the device holds at once (the
-    // family kernel's occupancy: registers and LDS), never more than items, so
-    // no block waits for a slot with a full share of items
-    b->nblocks = std::max(1, std::min(b->nitems, cus * 4));
     const void* fam_kernel[BF_COUNT] = {reinterpret_cast<const void*>(&k_batch<BF_REG>),
                                         reinterpret_cast<const void*>(&k_batch<BF_TTILE>),
                                         reinterpret_cast<const void*>(&k_batch<BF_BITS>),
-                                        reinterpret_cast<const void*>(&k_batch<BF_MARCH>)};
+                                        reinterpret_cast<const void*>(&k_batch<BF_J5>),
+                                        reinterpret_cast<const void*>(&k_batch<BF_BOX9>)};
     for (int f = 0; f < BF_COUNT; ++f) {
         int per_cu = 4;
-        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fam_kernel[f], kWave * kBatchWaves, 0);
-        b->fam_blocks[f] = std::max(1, std::min(b->fam_items[f], cus * std::max(1, per_cu)));
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fam_kernel[f], kWave * fam_waves(f), 0);
+        b->fam_slots[f] = cus * std::max(1, per_cu);
     }
+    count_items(b);
+    b->nblocks = std::max(1, std::min(b->nitems, cus * 4));
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
@@ -411,6 +498,7 @@ pskel_status_t pskel_batch_create(pskel_grid_t* const* grids, const pskel_stenci
     }
     if (e == hipSuccess) e = hipMalloc(&b->d_tab, b->host_tab.size() * sizeof(BatchEntry));
     if (e == hipSuccess) e = hipMalloc(&b->d_items, (size_t)b->nitems * sizeof(int));
+    if (e == hipSuccess) b->items_cap = (size_t)b->nitems;
     if (e != hipSuccess) {
         pskel_status_t st = hip_fail(e, "batch setup");
         pskel_batch_destroy(b);
@@ -457,9 +545,11 @@ pskel_status_t pskel_batch_run(pskel_batch_t* b, size_t iterations, int32_t use_
     for (pskel_grid_t* g : b->grids) PSKEL_HIP(hipStreamSynchronize(g->stream));
     pskel_status_t st;
     if (b->sched_sweeps != iterations) {
-        if ((st = plan_batch(b, iterations)) != PSKEL_OK) return st;
+        // the captured launches and the schedule go before their item list may
         if (b->exec) (void)hipGraphExecDestroy(b->exec);
         b->exec = nullptr;
+        b->sched_sweeps = 0;
+        if ((st = plan_batch(b, iterations)) != PSKEL_OK) return st;
     }
     if ((st = refresh_table(b)) != PSKEL_OK) return st;
     if (use_graph && (!b->exec || b->graph_sweeps != iterations)) {

@@ -55,30 +55,11 @@ static bool lt_depth_ok(int H, const RtPlan& q)
     return q.k >= 1 && q.k <= kLtMaxDepth && (H <= q.r * q.nw || 2 * q.k < q.r * q.nw);
 }
 
-// Tile shapes and the blocks of each that a CU holds, and the time of a launch in
-// microseconds: a launch, then rounds of blocks, each packing and unpacking its
-// rows and running its generations at the VALU's rate for the rows a CU holds
-// or, with few, at the latency of a barrier and one block's rows; no less than
-// its bytes take.  Fitted to 472 measured launches (64^2 to 8194^2, 1 to 30
-// generations): the fastest choice on all 8 boards.
+// Tile shapes and the blocks of each that a CU holds.
 struct LtShape {
     int r, nw, per_cu;
 };
 static constexpr LtShape kLtShapes[] = {{2, 8, 4}, {2, 16, 2}, {4, 16, 2}, {8, 8, 4}, {8, 16, 2}};
-
-static double lt_time(const LtShape& h, int W, int H, int k)
-{
-    constexpr double launch = 2.54, pack = 0.0442, row = 0.0093, barrier = 0.342, rate = 6.6e6;
-    constexpr int cus = 256;  // what the fit was measured on
-    const int rows = h.r * h.nw;
-    const int64_t nb = (int64_t)lt_tiles(W, kLtCols, 32) * lt_tiles(H, rows, k);
-    const int64_t slots = (int64_t)cus * h.per_cu, full = nb / slots, rest = nb % slots;
-    auto round = [&](int64_t b) {
-        return pack * (double)(b * rows) + k * std::max(row * (double)(b * rows), barrier + row * rows);
-    };
-    const double t = launch + (double)full * round(h.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0);
-    return std::max(t, launch + ((double)nb * kLtCols * rows + (double)W * H) / rate);
-}
 
 RtPlan life_tiles_plan(int W, int H, size_t rem, bool odd)
 {
@@ -91,7 +72,11 @@ RtPlan life_tiles_plan(int W, int H, size_t rem, bool odd)
             q.k = k;
             return lt_depth_ok(H, q);
         },
-        [&](const LtShape& h, int k) { return lt_time(h, W, H, k); });
+        [&](const LtShape& h, int k) {
+            const int rows = h.r * h.nw;
+            const int64_t nb = (int64_t)lt_tiles(W, kLtCols, 32) * lt_tiles(H, rows, k);
+            return lt_launch_time(rows, h.per_cu, nb, (double)W * H, k);
+        });
 }
 
 hipError_t launch_life_tiles(const Sweep2D& s, const RtPlan& q, hipStream_t st)

@@ -43,6 +43,24 @@ inline int lt_tiles(int n, int t, int h) { return n <= t ? 1 : 1 + (n - t + (t -
 // boards whose tiles (up to 256 rows) a 32-bit buffer offset covers
 inline bool lt_fits(size_t pitch) { return pitch * 256 < 0x7fffffffull; }
 
+// Time of one launch in microseconds: a launch, then rounds of blocks, each
+// packing and unpacking its rows and running its generations at the VALU's rate
+// for the rows a CU holds or, with few, at the latency of a barrier and one
+// block's rows; no less than its bytes take.  Fitted to 472 measured launches
+// (64^2 to 8194^2, 1 to 30 generations): the fastest choice on all 8 boards.
+// nb blocks of `rows` rows, per_cu of them on a CU at once, writing `cells` cells.
+inline double lt_launch_time(int rows, int per_cu, int64_t nb, double cells, int k)
+{
+    constexpr double launch = 2.54, pack = 0.0442, row = 0.0093, barrier = 0.342, rate = 6.6e6;
+    constexpr int cus = 256;  // what the fit was measured on
+    const int64_t slots = (int64_t)cus * per_cu, full = nb / slots, rest = nb % slots;
+    auto round = [&](int64_t b) {
+        return pack * (double)(b * rows) + k * std::max(row * (double)(b * rows), barrier + row * rows);
+    };
+    const double t = launch + (double)full * round(per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0);
+    return std::max(t, launch + ((double)nb * kLtCols * rows + cells) / rate);
+}
+
 #ifdef PSKEL_LTILE_INSTANTIATE
 namespace {
 

@@ -33,36 +33,13 @@ constexpr RtShape kRtShapes[] = {
     {PAT_CLOUD, 2, 8, 4}, {PAT_CLOUD, 2, 16, 2}, {PAT_CLOUD, 4, 8, 3},
 };
 
-// Time of one launch in microseconds: a launch, then rounds of blocks, each
-// sweep of a round at the VALU's rate for the rows a CU holds or, with few, at
-// the latency of a barrier and one block's rows; no less than its bytes take.
-// The constants are a least-squares fit of 820, 640 and 420 measured launches
-// (64^2 to 4096^2, depths 1 to 32): the fastest choice or one within 10% on 25
-// of 27 grids, 19% at worst.
-struct RtCost {
-    double launch, round, row, barrier, bytes;  // us, us, us per wave-row, us, bytes per us
-};
-constexpr RtCost rt_cost(int pattern)
-{
-    return pattern == PAT_J5     ? RtCost{3.30, 0.19, 0.0096, 0.272, 7.6e6}
-           : pattern == PAT_BOX9 ? RtCost{3.34, 0.00, 0.0269, 0.327, 6.2e6}
-                                 : RtCost{2.64, 1.39, 0.0316, 0.282, 7.2e6};
-}
-constexpr int kRtCus = 256;    // what the fit was measured on
 constexpr int kRtMaxDepth = 32;
 
 double rt_time(const RtShape& h, int W, int H, int k)
 {
-    const RtCost c = rt_cost(h.pattern);
     const int rows = h.r * h.nw;
     const int64_t nb = (int64_t)rt_tiles(W, kRtCols, rt_halo_cols(k)) * rt_tiles(H, rows, k);
-    const int64_t slots = (int64_t)kRtCus * h.per_cu, full = nb / slots, rest = nb % slots;
-    auto round = [&](int64_t b) {
-        return c.round + k * std::max(c.row * (double)(b * rows), c.barrier + c.row * rows);
-    };
-    const double t = c.launch + (double)full * round(h.per_cu) + (rest ? round((rest + kRtCus - 1) / kRtCus) : 0.0);
-    const double bytes = 4.0 * ((h.pattern == PAT_CLOUD ? 3.0 : 1.0) * (double)nb * kRtCols * rows + (double)W * H);
-    return std::max(t, c.launch + bytes / c.bytes);
+    return rt_launch_time(h.pattern, rows, h.per_cu, nb, (double)W * H, k);
 }
 
 }  // namespace

@@ -50,7 +50,7 @@ inline int rt_tiles(int n, int t, int h) { return n <= t ? 1 : 1 + (n - t + (t -
 // covers, wider than two lane vectors (a lane holds one ring column at most)
 inline bool rt_fits(int W, int H, size_t pitch)
 {
-    return W > 8 && H >= 3 && (uint64_t)(H + 512) * pitch * 4 < 0x7fffffffull;
+    return W > 8 && H >= 3 && (uint64_t)H * pitch * 4 < 0x7fffffffull && (uint64_t)(H + 256) * pitch * 4 < 0xffffffffull;
 }
 
 // what the stencils read besides the cells
@@ -61,6 +61,36 @@ struct RtParams {
     const float* wy;
     uint32_t fpitch;
 };
+
+// Time of one launch in microseconds: a launch, then rounds of blocks, each
+// sweep of a round at the VALU's rate for the rows a CU holds or, with few, at
+// the latency of a barrier and one block's rows; no less than its bytes take.
+// The constants are a least-squares fit of 820, 640 and 420 measured launches
+// (64^2 to 4096^2, depths 1 to 32): the fastest choice or one within 10% on 25
+// of 27 grids, 19% at worst.
+struct RtCost {
+    double launch, round, row, barrier, bytes;  // us, us, us per wave-row, us, bytes per us
+};
+constexpr RtCost rt_cost(int pattern)
+{
+    return pattern == PAT_J5     ? RtCost{3.30, 0.19, 0.0096, 0.272, 7.6e6}
+           : pattern == PAT_BOX9 ? RtCost{3.34, 0.00, 0.0269, 0.327, 6.2e6}
+                                 : RtCost{2.64, 1.39, 0.0316, 0.282, 7.2e6};
+}
+constexpr int kRtCus = 256;  // what the fit was measured on
+
+// nb blocks of `rows` rows, per_cu of them on a CU at once, writing `cells` cells
+inline double rt_launch_time(int pattern, int rows, int per_cu, int64_t nb, double cells, int k)
+{
+    const RtCost c = rt_cost(pattern);
+    const int64_t slots = (int64_t)kRtCus * per_cu, full = nb / slots, rest = nb % slots;
+    auto round = [&](int64_t b) {
+        return c.round + k * std::max(c.row * (double)(b * rows), c.barrier + c.row * rows);
+    };
+    const double t = c.launch + (double)full * round(per_cu) + (rest ? round((rest + kRtCus - 1) / kRtCus) : 0.0);
+    const double bytes = 4.0 * ((pattern == PAT_CLOUD ? 3.0 : 1.0) * (double)nb * kRtCols * rows + cells);
+    return std::max(t, c.launch + bytes / c.bytes);
+}
 
 #ifdef PSKEL_RTILE_INSTANTIATE
 namespace {

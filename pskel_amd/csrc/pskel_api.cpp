@@ -591,7 +591,7 @@ bool cloud_fields_fit(const pskel_grid_t* g)
         size_t fw, fh, fz, fp;
         const float* data;
         if (!field_info(g->fields[k], &fd, &fw, &fh, &fz, &data, &fp) ||
-            (uint64_t)(g->H + 512) * fp * 4 >= 0x7fffffffull)
+            (uint64_t)g->H * fp * 4 >= 0x7fffffffull || (uint64_t)(g->H + 256) * fp * 4 >= 0xffffffffull)
             return false;
     }
     return true;

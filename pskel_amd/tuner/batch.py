@@ -9,7 +9,9 @@ counterpart of the exhaustive search that judges the model: life at 1, 3, 5 or
 7 generations per launch, f32 at 1 or 3 sweeps in LDS tiles or 3 through the
 register march.  Every grid's tile at the chosen depth comes from the model.
 The timings run on scratch grids of the same shapes (the kernels' speed does
-not depend on the values), so the caller's grids are left as they are.
+not depend on the values), so the caller's grids are left as they are.  Above
+depth 1 the batch deepens a family's launches itself (pskel_batch_create), so
+the choices that differ are fused or not.
 
 The reference tunes one stencil at a time with GAlib
 (include/PSkelStencil.hpp:2014-2074); it has no batched launch.
