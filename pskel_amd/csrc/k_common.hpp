@@ -229,6 +229,18 @@ __device__ __forceinline__ float from_upper_lane(float v, float edge)
     return __uint_as_float(from_upper_lane(__float_as_uint(v), __float_as_uint(edge)));
 }
 
+// The same with zero where there is no source lane: the move folds into the
+// instruction that uses it.
+__device__ __forceinline__ float from_lower_lane0(float v)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), kDppWaveShr1, 0xf, 0xf, true));
+}
+
+__device__ __forceinline__ float from_upper_lane0(float v)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), kDppWaveShl1, 0xf, 0xf, true));
+}
+
 // ---------------------------------------------------------------------------
 // Deterministic FP64 block reduction: wave butterfly, then waves in order.
 // Every thread of the block must call it.  Returns the block sum in thread 0.

@@ -407,18 +407,25 @@ __global__ __launch_bounds__(NWD * NWW * kWave) void k3d_march2(Sweep3D s, float
                     for (int j = 0; j < VD; ++j) f[i][j] = LW::raw(w[i], j);
             }
         };
-        // a plane's boundary rows and edge cells into LDS
+        // a plane's boundary rows into LDS, and for 16-bit storage its edge cells
+        // (tiles of several waves along d; f32 puts those after all rows)
         auto stage = [&](LV (*L)[NL], float (*E)[NWD][RW][2], const float (&v)[RW][VD]) {
             lds_put<VD>(&L[2 * ww][col], v[0]);
             lds_put<VD>(&L[2 * ww + 1][col], v[RW - 1]);
-            if (lane == 0) {
+            if constexpr (!F32 && NWD > 1) {
+                if (lane == 0) {
 #pragma unroll
-                for (int i = 0; i < RW; ++i) E[ww][wd][i][0] = v[i][0];
-            }
-            if (lane == kWave - 1) {
+                    for (int i = 0; i < RW; ++i) E[ww][wd][i][0] = v[i][0];
+                }
+                if (lane == kWave - 1) {
 #pragma unroll
-                for (int i = 0; i < RW; ++i) E[ww][wd][i][1] = v[i][VD - 1];
+                    for (int i = 0; i < RW; ++i) E[ww][wd][i][1] = v[i][VD - 1];
+                }
             }
+        };
+        auto stage_edge = [&](float (*E)[NWD][RW][2], const float (&v)[RW][VD]) {
+#pragma unroll
+            for (int i = 0; i < RW; ++i) E[ww][wd][i][lane == 0 ? 0 : 1] = lane == 0 ? v[i][0] : v[i][VD - 1];
         };
         // one sweep at plane p on this lane's cells: lo/mid/hi hold planes p-1,
         // p, p+1 of its own rows; L/E plane p's boundary rows and edge cells.
@@ -451,8 +458,16 @@ __global__ __launch_bounds__(NWD * NWW * kWave) void k3d_march2(Sweep3D s, float
                     lds_get<VD>(&L[slot][col], wp);
                 }
                 // cells d-1 and d+VD: the neighbouring lane's, or across the wave edge
-                const float left = from_lower_lane(mid[i][VD - 1], E[ww][wd > 0 ? wd - 1 : 0][i][1]);
-                const float right = from_upper_lane(mid[i][0], E[ww][wd < NWD - 1 ? wd + 1 : NWD - 1][i][0]);
+                // (one wave along d: past the tile, never output, and the move folds
+                // into the add: 256^3 pair in f16 28.4 -> 26.1 us, in f32 33.8 -> 32.0)
+                float left, right;
+                if constexpr (NWD > 1) {
+                    left = from_lower_lane(mid[i][VD - 1], E[ww][wd > 0 ? wd - 1 : 0][i][1]);
+                    right = from_upper_lane(mid[i][0], E[ww][wd < NWD - 1 ? wd + 1 : NWD - 1][i][0]);
+                } else {
+                    left = from_lower_lane0(mid[i][VD - 1]);
+                    right = from_upper_lane0(mid[i][0]);
+                }
                 float val[VD];
 #pragma unroll
                 for (int j = 0; j < VD; ++j) {
@@ -539,13 +554,24 @@ __global__ __launch_bounds__(NWD * NWW * kWave) void k3d_march2(Sweep3D s, float
             }
 #pragma unroll
             for (int l = 0; l < NS; ++l) stage(ls[l][b], les[l][b], fs[l][I1]);
+            if (F32 && NWD > 1 && (lane == 0 || lane == kWave - 1)) {
+                stage_edge(lein[b], fin[I1]);
+#pragma unroll
+                for (int l = 0; l < NS; ++l) stage_edge(les[l][b], fs[l][I1]);
+            }
             __syncthreads();
             decode(in[I2], fin[I2]);  // plane h+1
+            // Where a sweep does not run, an f32 ring slot keeps an older plane (no
+            // output reads it): clearing it cost every step moves, taken or not
+            // (with the edge cells put once for all rows, depth 3 at 512^3: 251 us a
+            // launch cleared, 236 kept).  16-bit storage clears: kept planes spill
+            // there (bf16 pair 145 us, kept 258).
+            constexpr bool CLEAR = !F32;
             // sweep 1 at plane h (h >= ha: the loop starts there)
             if (h < min(h1 + NS, H)) {
                 sweep(std::true_type{}, h, fin[I0], fin[I1], fin[I2], in[I1], lin[b], lein[b], keys[0], sw[0][I2]);
                 decode(sw[0][I2], fs[0][I2]);
-            } else {
+            } else if constexpr (CLEAR) {
                 clear(sw[0][I2], fs[0][I2]);
             }
             // sweeps 2 .. DEPTH-1 at planes h-1 .. h-NS+1 (uniform bounds)
@@ -557,7 +583,7 @@ __global__ __launch_bounds__(NWD * NWW * kWave) void k3d_march2(Sweep3D s, float
                         sweep(std::false_type{}, q, fs[l - 1][I0], fs[l - 1][I1], fs[l - 1][I2], sw[l - 1][I1],
                               ls[l - 1][b], les[l - 1][b], keys[l], sw[l][I2]);
                         decode(sw[l][I2], fs[l][I2]);
-                    } else {
+                    } else if constexpr (CLEAR) {
                         clear(sw[l][I2], fs[l][I2]);
                     }
                 }
@@ -582,15 +608,26 @@ __global__ __launch_bounds__(NWD * NWW * kWave) void k3d_march2(Sweep3D s, float
                         }
                     }
                 }
+                if constexpr (F32) {
+                    const auto rs = plane_rsrc((T*)s.dst + (size_t)pl * plane, plane_bytes);
+#pragma unroll
+                    for (int i = 0; i < RW; ++i) buf_store<Word, NV>(rs, st_off[i], o[i]);
+                }
+            } else if constexpr (F32) {
+                // the same stores, discarded: the waits the compiler counts hold on both paths
+#pragma unroll
+                for (int i = 0; i < RW; ++i) buf_store<Word, NV>(plane_rsrc(s.dst, 0), kNoAccess, sw[0][I2][i]);
             } else {
 #pragma unroll
                 for (int i = 0; i < RW; ++i)
 #pragma unroll
                     for (int k = 0; k < NV; ++k) o[i][k] = Word(0);
             }
-            const auto rs = plane_rsrc((T*)s.dst + (size_t)(out2 ? pl : 0) * plane, out2 ? plane_bytes : 0);
+            if constexpr (!F32) {
+                const auto rs = plane_rsrc((T*)s.dst + (size_t)(out2 ? pl : 0) * plane, out2 ? plane_bytes : 0);
 #pragma unroll
-            for (int i = 0; i < RW; ++i) buf_store<Word, NV>(rs, st_off[i], o[i]);
+                for (int i = 0; i < RW; ++i) buf_store<Word, NV>(rs, st_off[i], o[i]);
+            }
             b ^= 1;
         };
         // whole rounds of NQ steps: a step past hend loads and stores through
