@@ -33,8 +33,6 @@ constexpr RtShape kRtShapes[] = {
     {PAT_CLOUD, 2, 8, 4}, {PAT_CLOUD, 2, 16, 2}, {PAT_CLOUD, 4, 8, 3},
 };
 
-constexpr int kRtMaxDepth = 32;
-
 double rt_time(const RtShape& h, int W, int H, int k)
 {
     const int rows = h.r * h.nw;
@@ -101,7 +99,7 @@ size_t rtile2d_blocks(int W, int H, const RtPlan& q)
 hipError_t launch_2d_rtile(const Sweep2D& s, const Points& pts, const CloudArgs* cloud, int pattern, const RtPlan& q,
                            double* partials, hipStream_t st)
 {
-    if (!rt_fits(s.W, s.H, s.pitch) || (partials && q.k != 1) || !rt_depth_ok(s.W, s.H, q)) return hipErrorInvalidValue;
+    if (!rt_fits(s.W, s.H, s.pitch) || !rt_depth_ok(s.W, s.H, q)) return hipErrorInvalidValue;
     RtParams p{};
     p.coeff = pts.coeff;
     for (int i = 0; i < 9; ++i) p.wt[i] = pts.wt[i];

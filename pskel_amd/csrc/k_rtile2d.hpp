@@ -174,8 +174,8 @@ __device__ __forceinline__ void rt_row(const RtParams& p, const float (&u)[4], c
 
 // Tile (tx, ty) of a grid tiled for K sweeps, by the block's NW waves; k sweeps
 // run (1 <= k <= K).  Every wave must call it (it synchronises the block).
-// With RES (k = 1) returns this lane's sum of squared changes over the tile's
-// own cells, ring cells included.
+// With RES returns this lane's sum of squared changes of the last sweep over the
+// tile's own cells, ring cells included.
 template <int PAT, int R, int NW, bool RES>
 __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, int tx, int ty, int K, int k, int lane,
                                           int wave, RtLds<R, NW>& L)
@@ -276,7 +276,9 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
 
     // One sweep: rows a[OLD .. OLD+R) -> a[NEW .. NEW+R).  The wave's end rows come
     // last, so that the neighbour waves' rows have left LDS by then.
-    auto sweep = [&](auto old_t, bool odd) __attribute__((always_inline)) {
+    // SUM: with RES, the last sweep.
+    auto sweep = [&](auto old_t, bool odd, auto sum_t) __attribute__((always_inline)) {
+        constexpr bool SUM = decltype(sum_t)::value;
         constexpr int OLD = decltype(old_t)::value, NEW = 1 - OLD;
         float ab[4], be[4];
         get(L.x[NEW][up][1], ab);
@@ -294,11 +296,13 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
                 rt_row<PAT>(p, u, c[i], d, 0.f, 0.f, rt_left(c[i]), rt_right(c[i]), 0.f, 0.f, fx[CLOUD ? i : 0],
                             fy[CLOUD ? i : 0], n[i]);
             }
-            if constexpr (RES) {
+            if constexpr (SUM) {
+                __builtin_amdgcn_sched_barrier(0);
                 if (edge) patch(i, odd, n[i]);
                 if (wy + i >= cy0 && wy + i < cy1) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
+                        __builtin_amdgcn_sched_barrier(0);
                         const double dv = (double)n[i][j] - (double)c[i][j];
                         if (xs + j >= cx0 && xs + j < cx1) rr += dv * dv;
                     }
@@ -323,7 +327,7 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
         row(R - 1, c[R - 2], be);
         sides(-1, ab);
         row(0, ab, c[1]);
-        if (!RES && edge) {  // no row reads another's new values: the ring goes back once
+        if (!SUM && edge) {  // no row reads another's new values: the ring goes back once
 #pragma unroll
             for (int i = 0; i < R; ++i) patch(i, odd, n[i]);
         }
@@ -362,23 +366,32 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
         for (; l < k; ++l) __syncthreads();
         return false;
     };
+    auto finish = [&](auto off_t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) store(i, a[i + decltype(off_t)::value]);
+        return rr;
+    };
+    constexpr std::integral_constant<int, 0> at0;
+    constexpr std::integral_constant<int, 1> at1;
     int l = 0;
+    // with RES the last sweep is another copy of the code: its sums, and the
+    // registers they take, stay out of the other sweeps
 #pragma unroll 1
     for (;;) {
         if (!exchange(l, L.x[0], a[1], a[R])) return rr;
-        sweep(std::integral_constant<int, 1>(), true);
-        if (RES || ++l == k) {
-#pragma unroll
-            for (int i = 0; i < R; ++i) store(i, a[i]);
-            return rr;
+        if (RES && l + 1 == k) {
+            sweep(at1, true, std::bool_constant<RES>());
+            return finish(at0);
         }
+        sweep(at1, true, std::false_type());
+        if (++l == k) return finish(at0);
         if (!exchange(l, L.x[1], a[0], a[R - 1])) return rr;
-        sweep(std::integral_constant<int, 0>(), false);
-        if (++l == k) {
-#pragma unroll
-            for (int i = 0; i < R; ++i) store(i, a[i + 1]);
-            return rr;
+        if (RES && l + 1 == k) {
+            sweep(at0, false, std::bool_constant<RES>());
+            return finish(at1);
         }
+        sweep(at0, false, std::false_type());
+        if (++l == k) return finish(at1);
     }
 }
 

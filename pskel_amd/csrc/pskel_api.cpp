@@ -413,10 +413,13 @@ struct RunPlan {
 
 // Sweeps fused in the next launch: up to the temporal depth, cut so that a launch
 // ends on every residual step.  The residual of sweep n is ||u^n - u^(n-1)||.
-// A 3D fused pair reduces it inside the launch (its second sweep against its
-// first); every other launch leaves only u^n and the state before the launch,
-// so in 2D a launch of k > 1 sweeps that would end on a residual step stops one
-// sweep short and the residual step runs as a single sweep.  A 2D launch of an
+// Fused 3D sweeps and 2D register tiles reduce it inside the launch (the last
+// sweep against the one before); every other launch leaves only u^n and the
+// state before the launch, so in 2D a launch of k > 1 sweeps that would end on a
+// residual step stops one sweep short and that step runs as a single sweep.
+// Reducing in the fused launch, us per 60 sweeps, before -> after, with a
+// residual every 20 and every 5: 9-point 1021 x 1531 166 -> 157, 270 -> 203;
+// 5-point 2048^2 147 -> 132, 331 -> 194.  A 2D launch of an
 // even number of sweeps writes a spare buffer; without one (odd2d) a launch
 // fuses one sweep less.
 // On register tiles the launch is as deep as rtile2d_plan makes it (*rt).
@@ -426,7 +429,8 @@ size_t next_k(const pskel::Grid& g, const RunPlan& plan, size_t done, size_t ite
     size_t k = plan.rtile ? iterations - done : std::min<size_t>((size_t)kmax, iterations - done);
     if (every) {
         k = std::min(k, (done / every + 1) * every - done);
-        if (g.ndim == 2 && k > 1 && (done + k) % every == 0) k -= 1;
+        const bool reduces = plan.rtile && plan.pattern != PAT_LIFE8;
+        if (g.ndim == 2 && !reduces && k > 1 && (done + k) % every == 0) k -= 1;
     }
     if (plan.rtile) {
         *rt = plan.pattern == PAT_LIFE8 ? life_tiles_plan((int)g.W, (int)g.H, k, g.odd_2d_launches)
@@ -435,6 +439,27 @@ size_t next_k(const pskel::Grid& g, const RunPlan& plan, size_t done, size_t ite
     }
     if (g.odd_2d_launches && g.ndim == 2 && k % 2 == 0) k -= 1;
     return k;
+}
+
+// FP64 partials of the register-tile launches that end on a residual step: the
+// last of those that cover an interval, which are the same in every interval.
+size_t rtile2d_partials(const pskel::Grid& g, const RunPlan& plan, const pskel_launch_cfg_t& cfg)
+{
+    if (!plan.rtile || plan.pattern == PAT_LIFE8 || cfg.residual_every <= 0) return 0;
+    const size_t every = (size_t)cfg.residual_every;
+    const int W = (int)g.W, H = (int)g.H;
+    size_t nb = 0;
+    if (every <= 4 * kRtMaxDepth) {
+        RtPlan q;
+        for (size_t done = 0; done < every; done += (size_t)q.k) (void)next_k(g, plan, done, every, 1, every, &q);
+        nb = rtile2d_blocks(W, H, q);
+    } else {  // any launch that may end a longer one
+        for (size_t k = 1; k <= kRtMaxDepth; ++k) {
+            const RtPlan q = rtile2d_plan(plan.pattern, W, H, k, g.odd_2d_launches);
+            if ((size_t)q.k == k) nb = std::max(nb, rtile2d_blocks(W, H, q));
+        }
+    }
+    return nb;
 }
 
 }  // namespace
@@ -486,6 +511,9 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
         }
         hipError_t e = hipSuccess;
         bool fused_res = false;
+        const bool reduces = want_res && plan.rtile && plan.pattern != PAT_LIFE8;
+        if (reduces && rtile2d_blocks((int)g->W, (int)g->H, rt) > g->partials_cap)
+            return fail(PSKEL_ERR_RUNTIME, "residual partials missing");
         // a temporal run's leftover single sweeps use the tuned kernel's own
         // default tile (tile_y/tile_z describe the temporal tile there)
         pskel_launch_cfg_t one = cfg;
@@ -509,7 +537,7 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
                 field_info(g->fields[0], &fd, &fw, &fh, &fz, &ca.wx, &ca.fpitch);
                 field_info(g->fields[1], &fd, &fw, &fh, &fz, &ca.wy, &ca.fpitch);
                 ca.dt = d.coeff;
-                if (plan.rtile) e = launch_2d_rtile(s, pts, &ca, plan.pattern, rt, want_res ? g->d_partials : nullptr, st);
+                if (plan.rtile) e = launch_2d_rtile(s, pts, &ca, plan.pattern, rt, reduces ? g->d_partials : nullptr, st);
                 else if (plan.path >= 1) e = launch_cloud_tuned(s, ca, one, st);
                 else e = launch_cloud_plain(s, ca, bx, by, st);
             } else if (g->storage == PSKEL_DTYPE_U8) {
@@ -519,14 +547,14 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
             } else {
                 if (plan.path == 3) e = launch_2d_points_f32(s, pts, st);
                 else if (plan.rtile)
-                    e = launch_2d_rtile(s, pts, nullptr, plan.pattern, rt, want_res ? g->d_partials : nullptr, st);
+                    e = launch_2d_rtile(s, pts, nullptr, plan.pattern, rt, reduces ? g->d_partials : nullptr, st);
                 else if (k > 1)
                     e = cfg.tile_x > 0 ? launch_2d_march_f32(s, pts, plan.pattern, (int)k, cfg, st)
                                        : launch_2d_ttile_f32(s, pts, plan.pattern, (int)k, cfg, st);
                 else if (plan.path >= 1) e = launch_2d_tuned_f32(s, pts, plan.pattern, one, st);
                 else e = launch_2d_plain_f32(s, pts, bx, by, st);
             }
-            if (plan.rtile && plan.pattern != PAT_LIFE8 && want_res && e == hipSuccess) {
+            if (reduces && e == hipSuccess) {
                 e = launch_reduce_partials(g->d_partials, rtile2d_blocks((int)g->W, (int)g->H, rt), g->d_res + nr, st);
                 fused_res = true;
             }
@@ -679,10 +707,7 @@ pskel_status_t plan_run(const pskel_grid_t* g, const pskel_stencil_desc_t* d, co
                      rtile2d_ok(plan.pattern, (int)g->W, (int)g->H, g->pitch) &&
                      (plan.pattern != PAT_CLOUD || cloud_fields_fit(g));
         // the allocation-free run's partials hold 65536 blocks
-        if (plan.rtile && plan.pattern != PAT_LIFE8 && g->odd_2d_launches && cfg.residual_every > 0 &&
-            rtile2d_blocks((int)g->W, (int)g->H, rtile2d_plan(plan.pattern, (int)g->W, (int)g->H, 1, true)) >
-                kScratchPartials)
-            plan.rtile = false;
+        if (plan.rtile && g->odd_2d_launches && rtile2d_partials(*g, plan, cfg) > kScratchPartials) plan.rtile = false;
         if (cfg.time_tile > 3 && ndim == 3) return fail(PSKEL_ERR_UNSUPPORTED, "3D temporal depth above 3");
         // two or three fused sweeps per launch run the 7-point Jacobi; for any
         // other 3D stencil the depth is a hint and sweeps run singly
@@ -733,10 +758,7 @@ namespace {
 size_t residual_partials(const pskel_grid_t* g, const RunPlan& plan, const Points& pts,
                          const pskel_launch_cfg_t& cfg)
 {
-    size_t nb = diff_blocks(g->nrows);
-    if (plan.rtile && plan.pattern != PAT_LIFE8)
-        nb = std::max(nb, rtile2d_blocks((int)g->W, (int)g->H,
-                                         rtile2d_plan(plan.pattern, (int)g->W, (int)g->H, 1, g->odd_2d_launches)));
+    size_t nb = std::max(diff_blocks(g->nrows), rtile2d_partials(*g, plan, cfg));
     if (g->ndim == 3 && plan.path == 3) {
         nb = std::max(nb, points3d_blocks(make_sweep3d(g, nullptr, nullptr, plan.radius, nullptr), pts));
     } else if (g->ndim == 3) {

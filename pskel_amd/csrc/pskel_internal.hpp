@@ -206,10 +206,11 @@ struct RtPlan {
     int r = 0, nw = 0, k = 0;
 };
 // The shape and depth with the least time for the run's remaining `rem` sweeps,
-// cut into launches of equal depth.  An even depth keeps the state's ring in
-// place (the next launch needs no ring copy); an odd one may end the run, and
-// is all there is without a spare buffer (odd).  Shape: {r, nw, ...}; ok(shape,
-// k): the tile is deep enough; time(shape, k): of one launch.
+// as launches of that depth and a shallower last one, then evened out.  An even
+// depth keeps the state's ring in place (the next launch needs no ring copy); an
+// odd one may end the run, and is all there is without a spare buffer (odd).
+// Shape: {r, nw, ...}; ok(shape, k): the tile is deep enough; time(shape, k): of
+// one launch.
 template <class Shape, size_t N, class Ok, class Time>
 RtPlan plan_fused(const Shape (&shapes)[N], size_t rem, bool odd, int kmax, Ok ok, Time time)
 {
@@ -220,7 +221,9 @@ RtPlan plan_fused(const Shape (&shapes)[N], size_t rem, bool odd, int kmax, Ok o
             if (!ok(h, k)) break;
             if ((size_t)k != rem && k != 1 && (k % 2 == 1) != odd) continue;
             if (odd && k % 2 == 0) continue;
-            const double t = time(h, k) * (double)((rem + k - 1) / k);
+            // launches of k and a shallower last one
+            const size_t whole = rem / k, tail = rem % k;
+            const double t = time(h, k) * (double)whole + (tail ? time(h, (int)tail) : 0.0);
             if (best.k && t >= best_t) continue;
             best.r = h.r;
             best.nw = h.nw;
@@ -236,11 +239,13 @@ RtPlan plan_fused(const Shape (&shapes)[N], size_t rem, bool odd, int kmax, Ok o
     return best;
 }
 
+constexpr int kRtMaxDepth = 32;  // sweeps of one launch, at most
+
 bool rtile2d_ok(int pattern, int W, int H, size_t pitch);
 // the next launch of a run with `rem` sweeps to go (odd: an odd number of them)
 RtPlan rtile2d_plan(int pattern, int W, int H, size_t rem, bool odd);
 size_t rtile2d_blocks(int W, int H, const RtPlan& q);
-// partials: with k = 1, one sum of squared changes per block
+// partials: one sum of the last sweep's squared changes per block
 hipError_t launch_2d_rtile(const Sweep2D& s, const Points& pts, const CloudArgs* cloud, int pattern, const RtPlan& q,
                            double* partials, hipStream_t st);
 
