@@ -637,8 +637,8 @@ PROFILES = {
     ("jacobi3d_single", "tuned"): "k3d_march_jacobi3d_512_f32.txt",
     ("jacobi3d_bf16", "tuned"): "k3d_march2_jacobi3d_512_bf16_stochastic.txt",
     ("jacobi3d_bf16_single", "tuned"): "k3d_march_jacobi3d_512_bf16_stochastic.txt",
-    ("life", "tuned"): "k_life_bits_life_8192_u8.txt",
-    ("jacobi2d", "tuned"): "k2d_march_jacobi2d_2048_f32.txt",
+    ("life", "tuned"): "k_life_tiles_life_8192_u8.txt",
+    ("jacobi2d", "tuned"): "k2d_rtile_jacobi2d_2048_f32.txt",
     ("diffusion9", "tuned"): "k2d_march_diffusion9_4096_f32.txt",
 }
 
@@ -652,8 +652,10 @@ def kernel_name(name, variant, launch):
     if name.startswith("jacobi3d"):
         return f"k3d_march2 (depth {k})" if k >= 2 else "k3d_march"
     if name == "life":
-        return f"k_life_bits (depth {k})" if k >= 2 else "k_life_tuned"
-    if name in ("jacobi2d", "diffusion9"):
+        return "k_life_tiles" if k >= 2 else "k_life_tuned"
+    if name == "jacobi2d":
+        return "k2d_rtile" if k >= 2 else "k2d_tuned"
+    if name == "diffusion9":  # 4096^2: above the register tiles' 12M cells
         if k >= 2:
             return f"k2d_march (depth {k})" if tile[0] == 4 else f"k2d_ttile (depth {k})"
         return "k2d_tuned"
