@@ -502,8 +502,8 @@ def measure_batch(steps, warmup, sweeps=200, compare=True, family_depths=None):
         "launch_steps": launches,
         "hbm_roofline_frac_per_sweep_bytes": nbytes * sweeps * steps / wall / (HBM_PEAK_GBS * 1e9),
         "depths": {str(k): depths.count(k) for k in sorted(set(depths))},
-        "f32_family": ("register march, 3 sweeps per launch, %d-row segments" % TB.MARCH_SEG
-                       if f32_choice == TB.MARCH else "LDS temporal tiles" if 3 in depths else "register tiles"),
+        "f32_family": ("fused sweeps on register tiles" if f32_choice == TB.MARCH or 3 in depths
+                       else "one-sweep tiles"),
         "march_grids": sum(1 for m in (march or []) if m),
         "items": info["items"],
         "persistent_blocks": info["blocks"],
