@@ -582,7 +582,9 @@ pskel_status_t pskel_batch_run(pskel_batch_t* b, size_t iterations, int32_t use_
     // the other buffer once per launch
     for (size_t i = 0; i < b->grids.size(); ++i) {
         pskel_grid_t* g = b->grids[i];
-        if (launches_of(b->host_tab[i]) % 2) advance_state(*g, 1);
+        const BatchEntry& e = b->host_tab[i];
+        if (launches_of(e) % 2) advance_state(*g, 1, e.radius);
+        else g->spare_width = std::min(g->spare_width, e.radius);
         g->sweeps_done += iterations;
     }
     if (stats) {

@@ -468,8 +468,11 @@ size_t rtile2d_partials(const pskel::Grid& g, const RunPlan& plan, const pskel_l
 // launch, wrote the other buffer: swap.  A 2D launch of even k wrote the spare
 // (the other buffer carries the other ring): the spare becomes current and
 // the old current becomes the spare.
-void pskel::advance_state(pskel::Grid& g, size_t k)
+// Sweeps at range r keep r rows and columns at each edge and write the cells
+// inside them, so the spare goes on holding at most r of its ring.
+void pskel::advance_state(pskel::Grid& g, size_t k, int radius)
 {
+    g.spare_width = std::min(g.spare_width, radius);
     if (k % 2 || g.ndim == 3) {
         std::swap(g.buf[0], g.buf[1]);
         g.parity ^= 1;
@@ -480,6 +483,19 @@ void pskel::advance_state(pskel::Grid& g, size_t k)
 }
 
 namespace {
+
+// the spare holds the ring that 2D sweeps at range `radius` from the current state keep
+bool spare_ring_ok(const pskel::Grid& g, int radius)
+{
+    return g.spare_parity == g.parity && g.spare_width >= radius;
+}
+
+void spare_ring_copied(pskel::Grid& g, int radius)
+{
+    if (spare_ring_ok(g, radius)) return;
+    g.spare_parity = g.parity;
+    g.spare_width = radius;
+}
 
 // Issue all launches for `iterations` sweeps; advances the grid state.
 pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Points& pts, size_t iterations,
@@ -502,10 +518,10 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
             dst = g->buf[1];
         } else {
             if (!g->buf[2]) return fail(PSKEL_ERR_RUNTIME, "spare buffer missing");
-            if (ndim == 2 && g->spare_parity != g->parity) {
+            if (!spare_ring_ok(*g, plan.radius)) {
                 Sweep2D rs = make_sweep2d(g, g->buf[0], g->buf[2], nullptr, plan.radius);
                 PSKEL_HIP(launch_copy_ring2d(rs, g->elem, st));
-                g->spare_parity = g->parity;
+                spare_ring_copied(*g, plan.radius);
             }
             dst = g->buf[2];
         }
@@ -585,7 +601,7 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
         }
         if (e != hipSuccess) return hip_fail(e, "stencil launch");
         nl++;
-        advance_state(*g, k);
+        advance_state(*g, k, plan.radius);
         g->sweeps_done += k;
         if (want_res) {
             if (!fused_res) {
@@ -1103,6 +1119,7 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
         PSKEL_HIP(hipMalloc(&g->buf[2], g->bytes));
         PSKEL_HIP(launch_copy(g->buf[2], g->buf[0], g->bytes, stream));
         g->spare_parity = g->parity;
+        g->spare_width = radius;
     }
 
     int64_t nl = 0, nr = 0;
@@ -1115,7 +1132,8 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
         // graph cache key: everything that shapes the launch sequence
         pskel_launch_cfg_t kc = cfg;
         kc.stream = nullptr;
-        const int sp = g->spare_parity * 2 + g->parity;
+        // which launches copy the spare's ring
+        const int sp = g->spare_parity * 4 + g->parity * 2 + (g->spare_width >= radius);
         const void* ptrs[5] = {g->buf[0], g->buf[1], g->buf[2], g->d_res, g->d_partials};
         // stochastic rounding bakes the sweep indices into the launches
         const uint64_t sweep0 = g->rounding == PSKEL_ROUND_STOCHASTIC ? g->sweeps_done : 0;
@@ -1178,8 +1196,8 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
         for (size_t done = 0; done < iterations;) {
             RtPlan rt;
             const size_t k = next_k(*g, plan, done, iterations, kmax, every, &rt);
-            if (k % 2 == 0 && g->ndim == 2) g->spare_parity = g->parity;  // ring copy in the graph
-            advance_state(*g, k);
+            if (k % 2 == 0 && g->ndim == 2) spare_ring_copied(*g, radius);  // ring copy in the graph
+            advance_state(*g, k, radius);
             g->sweeps_done += k;
             done += k;
         }
@@ -1342,6 +1360,7 @@ pskel_status_t pskel_grid_swap(pskel_grid_t* g)
     if (st != PSKEL_OK) return st;
     std::swap(g->buf[0], g->buf[1]);
     g->parity ^= 1;
+    g->spare_parity = -1;  // the caller's sweep may have written the ring too
     g->sweeps_done += 1;
     return PSKEL_OK;
 }

@@ -117,6 +117,7 @@ struct Grid {
     void* buf[3] = {nullptr, nullptr, nullptr}; // [cur, other, spare]
     int parity = 0;       // which uploaded buffer's ring `cur` carries (0 = input)
     int spare_parity = -1;// ring carried by the spare (-1: not allocated / unknown)
+    int spare_width = 0;  // rows and columns of that ring the spare carries
 
     hipStream_t stream = nullptr;
     bool own_stream = false;
@@ -131,7 +132,8 @@ struct Grid {
     bool odd_2d_launches = false;  // 2D launches fuse an odd number of sweeps (no spare buffer)
 };
 
-void advance_state(Grid& g, size_t k);
+// The ping-pong state after a launch of k sweeps at mask range `radius`.
+void advance_state(Grid& g, size_t k, int radius);
 
 // ---------------------------------------------------------------------------
 // Launch plumbing shared by the kernel TUs.
