@@ -213,8 +213,10 @@ pskel_status_t pskel_grid_upload(pskel_grid_t* grid, int32_t which, const void* 
                                  int32_t host_dtype);
 /* Copy the current state (the result of the last run) into a host array. */
 pskel_status_t pskel_grid_download(pskel_grid_t* grid, void* host, int32_t host_dtype);
-/* Copy the previous ping-pong state (the state one sweep before the result
- * when the last launch was a single sweep). */
+/* Copy the previous ping-pong state: the state one sweep before the result when
+ * the run, in launches of time_tile sweeps, ends in a single sweep (2D: on a
+ * residual step, when it leaves one sweep over after launches of time_tile, and
+ * always with CLOUDSIM); else an older state. */
 pskel_status_t pskel_grid_download_previous(pskel_grid_t* grid, void* host, int32_t host_dtype);
 pskel_status_t pskel_grid_info(const pskel_grid_t* grid, pskel_grid_info_t* info);
 
@@ -298,7 +300,8 @@ pskel_status_t pskel_tuner_host_search(const pskel_grid_desc_t* desc, const void
 pskel_status_t pskel_grid_swap(pskel_grid_t* grid);
 
 /* FP64 ||current - previous||_2 over every cell (the convergence test the
- * reference leaves to the caller). */
+ * reference leaves to the caller); `previous` as pskel_grid_download_previous
+ * copies it. */
 pskel_status_t pskel_grid_residual(pskel_grid_t* grid, double* out);
 
 /* ---- field arguments: Args / Args2D / Args3D (include/PSkelArgs.h:31-132,

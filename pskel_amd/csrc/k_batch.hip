@@ -157,8 +157,8 @@ __global__ __launch_bounds__(fam_waves(FAM) * kWave) void k_batch(const BatchEnt
                 p.coeff = E.coeff;
 #pragma unroll
                 for (int i = 0; i < 9; ++i) p.wt[i] = E.wt[i];
-                rt_tile<FAM == BF_J5 ? PAT_J5 : PAT_BOX9, kBatchTileRows, kBatchTileWaves, false>(s, p, tx, ty, E.depth, k,
-                                                                                                 lane, wave, L);
+                rt_tile<FAM == BF_J5 ? PAT_J5 : PAT_BOX9, kBatchTileRows, kBatchTileWaves, false, false>(
+                    s, p, tx, ty, E.depth, k, lane, wave, L);
             }
             __syncthreads();  // the next item's first rows go where this one's last may still be read
         } else {

@@ -175,8 +175,10 @@ __device__ __forceinline__ void rt_row(const RtParams& p, const float (&u)[4], c
 // Tile (tx, ty) of a grid tiled for K sweeps, by the block's NW waves; k sweeps
 // run (1 <= k <= K).  Every wave must call it (it synchronises the block).
 // With RES returns this lane's sum of squared changes of the last sweep over the
-// tile's own cells, ring cells included.
-template <int PAT, int R, int NW, bool RES>
+// tile's own cells, ring cells included.  With KEEP an even k also stores the state
+// before its last sweep in s.prev, if set (in the loop of every kernel the check
+// would cost the 5-point 8-row tiles a wave per SIMD).
+template <int PAT, int R, int NW, bool RES, bool KEEP>
 __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, int tx, int ty, int K, int k, int lane,
                                           int wave, RtLds<R, NW>& L)
 {
@@ -342,13 +344,13 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
     // the ring value it holds, which is dst's own, and cells past W land in the
     // row's padding (the pitch is a multiple of 256 cells)
     const bool own = xs >= cx0 && xs < cx1;
-    auto store = [&](int i, const float (&v)[4]) __attribute__((always_inline)) {
+    auto store = [&](const __amdgpu_buffer_rsrc_t& r, int i, const float (&v)[4]) __attribute__((always_inline)) {
         const int y = wy + i;
         if (y < cy0 || y >= cy1 || y < 1 || y > H - 2) return;  // uniform
         u32x4_t x;
 #pragma unroll
         for (int j = 0; j < 4; ++j) x[j] = __float_as_uint(v[j]);
-        __builtin_amdgcn_raw_buffer_store_b128(x, rd, (int)(own ? (uint32_t)y * pb + (uint32_t)xs * 4u : kNoAccess), 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(x, r, (int)(own ? (uint32_t)y * pb + (uint32_t)xs * 4u : kNoAccess), 0, 0);
     };
 
     // Level l's rows to the neighbour waves, and a barrier.  False: no later
@@ -368,8 +370,15 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
     };
     auto finish = [&](auto off_t) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < R; ++i) store(i, a[i + decltype(off_t)::value]);
+        for (int i = 0; i < R; ++i) store(rd, i, a[i + decltype(off_t)::value]);
         return rr;
+    };
+    // before the last of an even number of sweeps
+    auto keep_prev = [&]() __attribute__((always_inline)) {
+        if (!KEEP || !s.prev) return;  // uniform
+        const __amdgpu_buffer_rsrc_t rp = plane_rsrc(s.prev, bytes);
+#pragma unroll
+        for (int i = 0; i < R; ++i) store(rp, i, a[i]);
     };
     constexpr std::integral_constant<int, 0> at0;
     constexpr std::integral_constant<int, 1> at1;
@@ -387,23 +396,25 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
         if (++l == k) return finish(at0);
         if (!exchange(l, L.x[1], a[0], a[R - 1])) return rr;
         if (RES && l + 1 == k) {
+            keep_prev();
             sweep(at0, false, std::bool_constant<RES>());
             return finish(at1);
         }
+        if (KEEP && l + 1 == k) keep_prev();
         sweep(at0, false, std::false_type());
         if (++l == k) return finish(at1);
     }
 }
 
 // 64 registers (8 waves per SIMD, two blocks of 16 waves per CU) hold 4 rows
-template <int PAT, int R, int NW, bool RES>
+template <int PAT, int R, int NW, bool RES, bool KEEP>
 __global__ __launch_bounds__(NW * kWave, PAT != PAT_CLOUD && R <= 4 ? 8 : 1) void k2d_rtile(Sweep2D s, RtParams p, int ntx, int K, double* partials)
 {
     __shared__ RtLds<R, NW> L;
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int t = (int)xcd_remap(blockIdx.x, gridDim.x);
-    const double rr = rt_tile<PAT, R, NW, RES>(s, p, t % ntx, t / ntx, K, K, lane, wave, L);
+    const double rr = rt_tile<PAT, R, NW, RES, KEEP>(s, p, t % ntx, t / ntx, K, K, lane, wave, L);
     if constexpr (RES) {
         __shared__ double red[NW];
         const double v = block_sum<NW>(rr, red);

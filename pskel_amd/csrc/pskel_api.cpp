@@ -409,7 +409,22 @@ struct RunPlan {
     int pattern = PAT_GENERIC;
     int radius = 0;
     bool rtile = false;  // 2D fused sweeps on register tiles, as many per launch as pays
+    // the run leaves the state one sweep before its result in the other buffer,
+    // however deep its launches are (ends_single)
+    bool keep_prev = false;
 };
+
+// Does a 2D run end in a single sweep when it runs in launches of the depth it
+// names (field stencils: one sweep; a residual step is a single sweep)?  Then
+// download_previous and grid_residual after it read the state one sweep before
+// the result, and do so as well when the launches are deeper than that.
+bool ends_single(const RunPlan& plan, const pskel_launch_cfg_t& cfg, size_t iterations)
+{
+    const size_t every = cfg.residual_every > 0 ? (size_t)cfg.residual_every : 0;
+    if (plan.pattern == PAT_CLOUD || (every && iterations % every == 0)) return true;
+    const size_t last = every ? iterations % every : iterations;
+    return last % (size_t)cfg.time_tile == 1;
+}
 
 // Sweeps fused in the next launch: up to the temporal depth, cut so that a launch
 // ends on every residual step.  The residual of sweep n is ||u^n - u^(n-1)||.
@@ -422,7 +437,10 @@ struct RunPlan {
 // 5-point 2048^2 147 -> 132, 331 -> 194.  A 2D launch of an
 // even number of sweeps writes a spare buffer; without one (odd2d) a launch
 // fuses one sweep less.
-// On register tiles the launch is as deep as rtile2d_plan makes it (*rt).
+// On register tiles the launch is as deep as rtile2d_plan makes it (*rt).  A run
+// that keeps the state before its last sweep (keep_prev) ends in a single sweep or,
+// where the kernel can store that state beside its own result, in an even launch
+// (50 sweeps of CLOUDSIM at 4096^2: 719 us, with that store 733).
 size_t next_k(const pskel::Grid& g, const RunPlan& plan, size_t done, size_t iterations, int kmax, size_t every,
               RtPlan* rt)
 {
@@ -433,6 +451,8 @@ size_t next_k(const pskel::Grid& g, const RunPlan& plan, size_t done, size_t ite
         if (g.ndim == 2 && !reduces && k > 1 && (done + k) % every == 0) k -= 1;
     }
     if (plan.rtile) {
+        const bool stores = plan.pattern == PAT_CLOUD || (every && (done + k) % every == 0);
+        if (plan.keep_prev && k > 1 && done + k == iterations && (!stores || k % 2 == 1)) k -= 1;
         *rt = plan.pattern == PAT_LIFE8 ? life_tiles_plan((int)g.W, (int)g.H, k, g.odd_2d_launches)
                                         : rtile2d_plan(plan.pattern, (int)g.W, (int)g.H, k, g.odd_2d_launches);
         return (size_t)rt->k;
@@ -443,8 +463,9 @@ size_t next_k(const pskel::Grid& g, const RunPlan& plan, size_t done, size_t ite
 
 // FP64 partials of the register-tile launches that end on a residual step: the
 // last of those that cover an interval, which are the same in every interval.
-size_t rtile2d_partials(const pskel::Grid& g, const RunPlan& plan, const pskel_launch_cfg_t& cfg)
+size_t rtile2d_partials(const pskel::Grid& g, RunPlan plan, const pskel_launch_cfg_t& cfg)
 {
+    plan.keep_prev = false;  // an interval that is not the run's last
     if (!plan.rtile || plan.pattern == PAT_LIFE8 || cfg.residual_every <= 0) return 0;
     const size_t every = (size_t)cfg.residual_every;
     const int W = (int)g.W, H = (int)g.H;
@@ -453,6 +474,8 @@ size_t rtile2d_partials(const pskel::Grid& g, const RunPlan& plan, const pskel_l
         RtPlan q;
         for (size_t done = 0; done < every; done += (size_t)q.k) (void)next_k(g, plan, done, every, 1, every, &q);
         nb = rtile2d_blocks(W, H, q);
+        // with keep_prev the run's last interval ends the same way or in a single sweep
+        if (!g.odd_2d_launches) nb = std::max(nb, rtile2d_blocks(W, H, rtile2d_plan(plan.pattern, W, H, 1, false)));
     } else {  // any launch that may end a longer one
         for (size_t k = 1; k <= kRtMaxDepth; ++k) {
             const RtPlan q = rtile2d_plan(plan.pattern, W, H, k, g.odd_2d_launches);
@@ -544,6 +567,7 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
         }
         if (ndim == 2) {
             Sweep2D s = make_sweep2d(g, src, dst, g->buf[1], plan.radius);
+            if (plan.keep_prev && inplace && done + k == iterations) s.prev = g->buf[1];
             const int bx = cfg.block_x > 0 ? cfg.block_x : 64;
             const int by = cfg.block_y > 0 ? cfg.block_y : 4;
             if (plan.pattern == PAT_CLOUD) {
@@ -1096,6 +1120,7 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
     const int radius = plan.radius;
     if (stats) stats->sweeps = (int64_t)iterations;
     if (iterations == 0) return PSKEL_OK;
+    plan.keep_prev = plan.rtile && ends_single(plan, cfg, iterations);
 
     PSKEL_HIP(hipSetDevice(g->device));
     hipStream_t stream = cfg.stream ? (hipStream_t)cfg.stream : g->stream;

@@ -145,6 +145,8 @@ struct Sweep2D {
     int W, H;
     size_t pitch;
     int radius;
+    void* prev = nullptr;   // register tiles with partials or of CLOUDSIM, even depths: the state before
+                            // the last sweep goes here too
 };
 
 struct Sweep3D {
