@@ -353,7 +353,9 @@ pskel_status_t pskel_grid_set_field(pskel_grid_t* grid, int32_t slot, pskel_fiel
  *      at a wider range runs LDS tiles of tile_y rows (16 or 32; default 16).
  *      A launch fuses an odd number k, so it moves a grid's state to its other
  *      buffer: N sweeps run as N / k launches of k and the rest as one odd
- *      launch or two (r - 1, then 1).  At depth 1 cfgs[i].tile_y is the rows
+ *      launch or two (r - 1, then 1); a grid whose launches of k = time_tile
+ *      would end in a single sweep ends in one at any depth, so that its
+ *      previous state is the one before it.  At depth 1 cfgs[i].tile_y is the rows
  *      per lane (1, 2, 4, 8; default 4).  tile_x = 4 at depth 3 (the register
  *      march's launch) is accepted for grids over 8 cells wide and runs the
  *      same register tiles.  cfgs may be NULL (depth 1, 4 rows). */

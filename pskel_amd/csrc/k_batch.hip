@@ -21,7 +21,9 @@
 // per launch moves the state to the other buffer, so grid g's launch l reads
 // buffer l & 1 and writes the other, with no third buffer.  N sweeps of grid g
 // run as N / K launches of K, then the rest r = N mod K as one launch of r
-// (odd) or two of r - 1 and 1 (even r): n_g launches.  Work items are ordered by
+// (odd) or two of r - 1 and 1 (even r): n_g launches.  Where launches of the depth
+// asked for end in a single sweep, so do these (N - 1 sweeps as above, then 1): the
+// other buffer then holds the state before it.  Work items are ordered by
 // n_g, longest first, so launch l's items are a prefix of the list.
 #include <algorithm>
 #include <cstring>
@@ -52,7 +54,7 @@ struct BatchEntry {
     int rtile;        // f32 at K = 3 on register tiles
     int depth;        // K, sweeps fused per launch (odd); of a tile family: the tiles' halo
     int full;         // launches of K sweeps
-    int tail0, tail1; // sweeps of the launches after them (odd; 0: none)
+    int tail0, tail1, tail2;  // sweeps of the launches after them (odd; 0: none)
     int tiles_x;      // tiles along w
     int ntiles;       // tiles of the grid
     int item0;        // first work item of this grid
@@ -75,6 +77,7 @@ __device__ __forceinline__ int sweeps_of(const BatchEntry& E, int launch)
     if (launch < E.full) return E.depth;
     if (launch == E.full) return E.tail0;
     if (launch == E.full + 1) return E.tail1;
+    if (launch == E.full + 2) return E.tail2;
     return 0;
 }
 
@@ -176,18 +179,27 @@ int family_of(const BatchEntry& e)
     return BF_TTILE;
 }
 
-// the schedule of N sweeps at depth K: full launches of K, then the tail
-void schedule(BatchEntry& e, size_t n)
+// the schedule of N sweeps at depth K: full launches of K, then the tail; it ends in
+// a single sweep where the schedule at depth `asked` does
+void schedule(BatchEntry& e, size_t n, int asked)
 {
     const int K = e.depth;
-    e.full = (int)(n / K);
-    const int r = (int)(n % K);
-    e.tail0 = e.tail1 = 0;
-    if (r % 2 == 1) e.tail0 = r;
-    else if (r > 0) {
-        e.tail0 = r - 1;
-        e.tail1 = 1;
-    }
+    auto split = [&](size_t m) {
+        e.full = (int)(m / K);
+        const int r = (int)(m % K);
+        e.tail0 = e.tail1 = e.tail2 = 0;
+        if (r % 2 == 1) e.tail0 = r;
+        else if (r > 0) {
+            e.tail0 = r - 1;
+            e.tail1 = 1;
+        }
+    };
+    split(n);
+    const size_t rest = n % (size_t)asked;
+    const bool single = asked == 1 || rest == 1 || (rest > 0 && rest % 2 == 0);
+    if (!single || (e.tail1 ? e.tail1 : e.tail0 ? e.tail0 : K) == 1) return;
+    split(n - 1);
+    (e.tail0 == 0 ? e.tail0 : e.tail1 == 0 ? e.tail1 : e.tail2) = 1;
 }
 
 // tiles of a grid of a register-tile family at depth K
@@ -202,7 +214,7 @@ void tile_grid(BatchEntry& e, int K)
     e.ntiles = e.tiles_x * rt_tiles(e.H, kBatchTileH, K);
 }
 
-int launches_of(const BatchEntry& e) { return e.full + (e.tail0 > 0) + (e.tail1 > 0); }
+int launches_of(const BatchEntry& e) { return e.full + (e.tail0 > 0) + (e.tail1 > 0) + (e.tail2 > 0); }
 
 }  // namespace
 
@@ -286,7 +298,7 @@ int family_depth(const pskel_batch_t* b, int f, size_t n)
         }
         BatchEntry t{};
         t.depth = K;
-        schedule(t, n);
+        schedule(t, n, lo);
         const int per_cu = std::max(1, b->fam_slots[f] / kRtCus);
         const double one = life ? lt_launch_time(kBatchTileH, per_cu, nb, cells, K)
                                 : rt_launch_time(f == BF_J5 ? PAT_J5 : PAT_BOX9, kBatchTileH, per_cu, nb, cells, K);
@@ -319,7 +331,7 @@ pskel_status_t plan_batch(pskel_batch_t* b, size_t n)
         PSKEL_HIP(hipMalloc(&b->d_items, (size_t)b->nitems * sizeof(int)));
         b->items_cap = (size_t)b->nitems;
     }
-    for (auto& e : b->host_tab) schedule(e, n);
+    for (size_t i = 0; i < ng; ++i) schedule(b->host_tab[i], n, b->asked[i]);
     std::vector<int> order(ng);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(),
