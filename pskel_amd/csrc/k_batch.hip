@@ -16,9 +16,9 @@
 // the LDS temporal tile; 1, 3, 5 or 7 for life, on bit-packed tiles
 // (k_ltile.hpp); K = 1 runs the one-sweep tiles of k_tiles2d.hpp).  A grid of
 // a family that holds its tiles in registers (bit-packed life, the f32 register
-// tiles) fuses as many sweeps as pay for the whole family, at least the depth
-// asked for: plan_batch picks it for each run length.  An odd number of sweeps
-// per launch moves the state to the other buffer, so grid g's launch l reads
+// tiles) fuses as many sweeps as pay for the whole family, at least the depths
+// its grids ask for: plan_batch picks it for each run length.  An odd number of
+// sweeps per launch moves the state to the other buffer, so grid g's launch l reads
 // buffer l & 1 and writes the other, with no third buffer.  N sweeps of grid g
 // run as N / K launches of K, then the rest r = N mod K as one launch of r
 // (odd) or two of r - 1 and 1 (even r): n_g launches.  Where launches of the depth
@@ -265,8 +265,8 @@ void count_items(pskel_batch_t* b)
     }
 }
 
-// The depth of a register-tile family for runs of n sweeps: odd, at least the
-// least one asked for and at most n, with the least time for the run's launches
+// The depth of a register-tile family for runs of n sweeps: odd, at least what
+// each of its grids asked for and at most n, with the least time for the run's launches
 // (the tiles' halo grows with it, the crossings of memory and the launches get
 // fewer).  A batched launch costs about 8 us more than one of a single grid (the
 // item and table lookups, the graph's steps).  Measured, 105 sweeps of the f32
@@ -283,7 +283,7 @@ int family_depth(const pskel_batch_t* b, int f, size_t n)
     for (size_t i = 0; i < b->host_tab.size(); ++i) {
         const BatchEntry& e = b->host_tab[i];
         if (family_of(e) != f) continue;
-        lo = lo ? std::min(lo, b->asked[i]) : b->asked[i];
+        lo = std::max(lo, b->asked[i]);
         cells += (double)e.W * e.H;
     }
     int best = lo;
