@@ -97,8 +97,8 @@ __global__ __launch_bounds__(1024) void k2d_cloud_plain(Sweep2D s, CloudArgs a)
     const float* __restrict__ in = (const float*)s.src;
     const size_t p = s.pitch;
     const size_t i = (size_t)h * p + w;
-    const size_t f = (size_t)h * a.fpitch + w;
-    ((float*)s.dst)[i] = cloud_cell(in[i], in[i - p], in[i + 1], in[i - 1], in[i + p], a.wx[f], a.wy[f], a.dt);
+    const float xw = a.wx[(size_t)h * a.xpitch + w], yw = a.wy[(size_t)h * a.ypitch + w];
+    ((float*)s.dst)[i] = cloud_cell(in[i], in[i - p], in[i + 1], in[i - 1], in[i + p], xw, yw, a.dt);
 }
 
 // 64 lanes x float4 = 256 columns per wave, RY rows per lane, waves stacked
@@ -140,8 +140,8 @@ __global__ __launch_bounds__(256) void k2d_cloud_tuned(Sweep2D s, CloudArgs a)
         fx[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         fy[i] = fx[i];
         if (col_live && h >= 1 && h < H - 1) {
-            fx[i] = *reinterpret_cast<const float4*>(a.wx + (size_t)h * a.fpitch + w);
-            fy[i] = *reinterpret_cast<const float4*>(a.wy + (size_t)h * a.fpitch + w);
+            fx[i] = *reinterpret_cast<const float4*>(a.wx + (size_t)h * a.xpitch + w);
+            fy[i] = *reinterpret_cast<const float4*>(a.wy + (size_t)h * a.ypitch + w);
         }
     }
     float lf[RY + 2], rt[RY + 2];

@@ -115,7 +115,8 @@ hipError_t launch_2d_rtile(const Sweep2D& s, const Points& pts, const CloudArgs*
         p.coeff = cloud->dt;
         p.wx = cloud->wx;
         p.wy = cloud->wy;
-        p.fpitch = (uint32_t)cloud->fpitch;
+        p.xpitch = (uint32_t)cloud->xpitch;
+        p.ypitch = (uint32_t)cloud->ypitch;
     }
     if (pattern == PAT_J5) return rt_shape<PAT_J5>(s, p, q, partials, st);
     if (pattern == PAT_BOX9) return rt_shape<PAT_BOX9>(s, p, q, partials, st);

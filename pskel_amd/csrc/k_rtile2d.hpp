@@ -57,9 +57,9 @@ inline bool rt_fits(int W, int H, size_t pitch)
 struct RtParams {
     float coeff;         // 5-point: the scale; CLOUDSIM: the time step
     float wt[9];         // 3x3 weights
-    const float* wx;     // CLOUDSIM's fields, rows of fpitch
+    const float* wx;     // CLOUDSIM's fields, rows of xpitch and ypitch
     const float* wy;
-    uint32_t fpitch;
+    uint32_t xpitch, ypitch;
 };
 
 // Time of one launch in microseconds: a launch, then rounds of blocks, each
@@ -203,13 +203,13 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
     for (int i = 0; i < R; ++i) rt_load(rs, roff(wy + i), a[i + 1]);
     float fx[CLOUD ? R : 1][4], fy[CLOUD ? R : 1][4];
     if constexpr (CLOUD) {
-        const int fbytes = (int)((uint32_t)H * p.fpitch * 4u);
-        const __amdgpu_buffer_rsrc_t rx = plane_rsrc(p.wx, fbytes), ry = plane_rsrc(p.wy, fbytes);
+        const uint32_t xb = p.xpitch * 4u, yb = p.ypitch * 4u;
+        const __amdgpu_buffer_rsrc_t rx = plane_rsrc(p.wx, (int)((uint32_t)H * xb));
+        const __amdgpu_buffer_rsrc_t ry = plane_rsrc(p.wy, (int)((uint32_t)H * yb));
 #pragma unroll
         for (int i = 0; i < R; ++i) {
-            const uint32_t o = xs < W ? (uint32_t)(wy + i) * p.fpitch * 4u + (uint32_t)xs * 4u : kNoAccess;
-            rt_load(rx, o, fx[i]);
-            rt_load(ry, o, fy[i]);
+            rt_load(rx, xs < W ? (uint32_t)(wy + i) * xb + (uint32_t)xs * 4u : kNoAccess, fx[i]);
+            rt_load(ry, xs < W ? (uint32_t)(wy + i) * yb + (uint32_t)xs * 4u : kNoAccess, fy[i]);
         }
     }
 

@@ -574,8 +574,8 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
                 CloudArgs ca;
                 int fd;
                 size_t fw, fh, fz;
-                field_info(g->fields[0], &fd, &fw, &fh, &fz, &ca.wx, &ca.fpitch);
-                field_info(g->fields[1], &fd, &fw, &fh, &fz, &ca.wy, &ca.fpitch);
+                field_info(g->fields[0], &fd, &fw, &fh, &fz, &ca.wx, &ca.xpitch);
+                field_info(g->fields[1], &fd, &fw, &fh, &fz, &ca.wy, &ca.ypitch);
                 ca.dt = d.coeff;
                 if (plan.rtile) e = launch_2d_rtile(s, pts, &ca, plan.pattern, rt, reduces ? g->d_partials : nullptr, st);
                 else if (plan.path >= 1) e = launch_cloud_tuned(s, ca, one, st);

@@ -175,11 +175,11 @@ inline float scaled_sum_offset_term(float coeff, int npoints, float off)
 }
 
 // CLOUDSIM field arguments as its kernels see them (reversed device layout:
-// the field value of cell (h, w) at h*fpitch + w).
+// the field value of cell (h, w) at h*pitch + w, each field with its own pitch).
 struct CloudArgs {
     const float* wx;
     const float* wy;
-    size_t fpitch;
+    size_t xpitch, ypitch;
     float dt;
 };
 
