@@ -1141,10 +1141,18 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
         for (int k = 2; k <= std::max(2, cfg.time_tile); ++k) (void)ttile3d_blocks(s3, g->storage, cfg, k);
     }
     if ((plan.path == 2 || plan.rtile) && ndim == 2 && !g->buf[2]) {
-        PSKEL_HIP(hipMalloc(&g->buf[2], g->bytes));
-        PSKEL_HIP(launch_copy(g->buf[2], g->buf[0], g->bytes, stream));
-        g->spare_parity = g->parity;
-        g->spare_width = radius;
+        const hipError_t e = hipMalloc(&g->buf[2], g->bytes);
+        if (e == hipSuccess) {
+            PSKEL_HIP(launch_copy(g->buf[2], g->buf[0], g->bytes, stream));
+            g->spare_parity = g->parity;
+            g->spare_width = radius;
+        } else {
+            g->buf[2] = nullptr;
+            // field stencils need no spare for single sweeps
+            if (plan.path == 2) return hip_fail(e, "spare buffer");
+            (void)hipGetLastError();
+            plan.rtile = plan.keep_prev = false;
+        }
     }
 
     int64_t nl = 0, nr = 0;
