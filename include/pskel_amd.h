@@ -255,8 +255,10 @@ pskel_status_t pskel_run_iterative_host(const pskel_grid_desc_t* desc, const voi
  *      buffer holds nrows rows of `pitch` elements (nrows = height in 2D,
  *      height*width in 3D; row h (2D) or (h, w) (3D) at row*pitch); pitch must
  *      cover a row (width in 2D, depth in 3D) and be a whole number of 1 KiB;
- *      both buffers 256-byte aligned.  `in` is the initial state and is
- *      overwritten with intermediate states, as runIterativeCPU overwrites
+ *      both buffers 256-byte aligned.  2D sweeps leave the rows' padding alone,
+ *      but for the register march (up to 3 cells past a row's end) and the
+ *      copy of the whole buffer when a run ends in `in`.  `in` is the initial
+ *      state and is overwritten with intermediate states, as runIterativeCPU does with
  *      `input` (include/PSkelStencil.hpp:903-932); the result of the
  *      iterations is left in `out` (iterations == 0 copies `in`).  2D
  *      temporal tiles fuse an odd number of sweeps per launch (even depths

@@ -245,9 +245,13 @@ __device__ __forceinline__ void life_tile(const Sweep2D& s, int tx, int ty, int 
     }
 
     // the tile's own interior rows; a lane holding a ring column writes the ring
-    // value it holds, which is dst's own, and cells past W land in the padding
+    // value it holds, which is dst's own.  The padding of a row may be the caller's:
+    // a 16-byte half that reaches past W is stored in pieces of 8, 4, 2 and 1 cells.
     const __amdgpu_buffer_rsrc_t rd = plane_rsrc((uint8_t*)s.dst + (size_t)y0 * pitch, bytes);
     const bool own = xs >= cx0 && xs < cx1;
+    const int cells = own ? min(W - xs, 32) : 0;          // this lane's cells on the board
+    const bool ragged = W % 16 != 0 && x0 + kLtCols >= W;  // uniform
+    const int part = ragged ? cells & 15 : 0;              // cells of such a half
 #pragma unroll
     for (int i = 0; i < R; ++i) {
         const int y = wy + i;
@@ -258,9 +262,21 @@ __device__ __forceinline__ void life_tile(const Sweep2D& s, int tx, int ty, int 
             a[q] = lt_unpack(c[i], q);
             b[q] = lt_unpack(c[i], q + 4);
         }
-        const uint32_t o = own ? off(i) : kNoAccess;
-        __builtin_amdgcn_raw_buffer_store_b128(a, rd, (int)o, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(b, rd, (int)o + 16, 0, 0);
+        const uint32_t o = off(i);
+        __builtin_amdgcn_raw_buffer_store_b128(a, rd, (int)(cells >= 16 ? o : kNoAccess), 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(b, rd, (int)(cells == 32 ? o + 16 : kNoAccess), 0, 0);
+        if (!ragged) continue;
+        const uint32_t h = o + (cells & 16);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] = cells & 16 ? b[q] : a[q];
+        const u32x2_t two = {a[0], a[1]};
+        __builtin_amdgcn_raw_buffer_store_b64(two, rd, (int)(part & 8 ? h : kNoAccess), 0, 0);
+        const uint32_t w4 = part & 8 ? a[2] : a[0];
+        __builtin_amdgcn_raw_buffer_store_b32(w4, rd, (int)(part & 4 ? h + (part & 8) : kNoAccess), 0, 0);
+        const uint32_t w2 = part & 8 ? (part & 4 ? a[3] : a[2]) : (part & 4 ? a[1] : a[0]);
+        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)w2, rd, (int)(part & 2 ? h + (part & 12) : kNoAccess), 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(part & 2 ? w2 >> 16 : w2), rd,
+                                             (int)(part & 1 ? h + (part & 14) : kNoAccess), 0, 0);
     }
 }
 

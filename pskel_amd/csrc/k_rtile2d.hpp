@@ -340,17 +340,40 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
     };
 
     const __amdgpu_buffer_rsrc_t rd = plane_rsrc(s.dst, bytes);
+    const bool own_x = xs >= cx0 && xs < cx1;
     // the tile's own interior rows; a lane vector holding a ring column writes
-    // the ring value it holds, which is dst's own, and cells past W land in the
-    // row's padding (the pitch is a multiple of 256 cells)
-    const bool own = xs >= cx0 && xs < cx1;
-    auto store = [&](const __amdgpu_buffer_rsrc_t& r, int i, const float (&v)[4]) __attribute__((always_inline)) {
-        const int y = wy + i;
-        if (y < cy0 || y >= cy1 || y < 1 || y > H - 2) return;  // uniform
-        u32x4_t x;
+    // the ring value it holds, which is dst's own.  The padding of a row may be
+    // the caller's (not CLOUDSIM's, whose buffers are a grid's): the vector that
+    // reaches past W stores its cells as a pair and a single.
+    auto store = [&](const __amdgpu_buffer_rsrc_t& r, auto off_t) __attribute__((always_inline)) {
+        // 5-point and 9-point: recomputed from the lane; hoisted above the sweeps,
+        // these would hold registers there (5-point 8-row tiles 81 for 72, two waves
+        // per SIMD less)
+        int x = xs;
+        bool own = own_x;
+        if constexpr (!CLOUD) {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));
+            x = x0 + ln * 4;
+            own = x >= cx0 && x < cx1;
+        }
+        const bool ragged = !CLOUD && W % 4 != 0 && x0 + kRtCols >= W;  // uniform
+        const int part = ragged && own && x + 4 > W ? W - x : 0;  // cells of such a vector
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x[j] = __float_as_uint(v[j]);
-        __builtin_amdgcn_raw_buffer_store_b128(x, r, (int)(own ? (uint32_t)y * pb + (uint32_t)xs * 4u : kNoAccess), 0, 0);
+        for (int i = 0; i < R; ++i) {
+            const int y = wy + i;
+            if (y < cy0 || y >= cy1 || y < 1 || y > H - 2) continue;  // uniform
+            const uint32_t o = (uint32_t)y * pb + (uint32_t)x * 4u;
+            u32x4_t v;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = __float_as_uint(a[i + decltype(off_t)::value][j]);
+            __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)(own && !part ? o : kNoAccess), 0, 0);
+            if (!ragged) continue;
+            const u32x2_t two = {v[0], v[1]};
+            __builtin_amdgcn_raw_buffer_store_b64(two, r, (int)(part & 2 ? o : kNoAccess), 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(part & 2 ? v[2] : v[0], r,
+                                                  (int)(part & 1 ? o + (part & 2) * 4u : kNoAccess), 0, 0);
+        }
     };
 
     // Level l's rows to the neighbour waves, and a barrier.  False: no later
@@ -368,20 +391,17 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
         for (; l < k; ++l) __syncthreads();
         return false;
     };
+    constexpr std::integral_constant<int, 0> at0;
+    constexpr std::integral_constant<int, 1> at1;
     auto finish = [&](auto off_t) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < R; ++i) store(rd, i, a[i + decltype(off_t)::value]);
+        store(rd, off_t);
         return rr;
     };
     // before the last of an even number of sweeps
     auto keep_prev = [&]() __attribute__((always_inline)) {
         if (!KEEP || !s.prev) return;  // uniform
-        const __amdgpu_buffer_rsrc_t rp = plane_rsrc(s.prev, bytes);
-#pragma unroll
-        for (int i = 0; i < R; ++i) store(rp, i, a[i]);
+        store(plane_rsrc(s.prev, bytes), at0);
     };
-    constexpr std::integral_constant<int, 0> at0;
-    constexpr std::integral_constant<int, 1> at1;
     int l = 0;
     // with RES the last sweep is another copy of the code: its sums, and the
     // registers they take, stay out of the other sweeps
