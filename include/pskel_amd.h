@@ -396,7 +396,9 @@ pskel_status_t pskel_tuner_candidates(const pskel_tune_query_t* q, const pskel_s
 /* Model input of one (query, descriptor, candidate): PSKEL_TUNER_NFEAT floats. */
 pskel_status_t pskel_tuner_features(const pskel_tune_query_t* q, const pskel_stencil_desc_t* d,
                                     const pskel_launch_cfg_t* c, float* feat);
-/* The candidate with the lowest predicted time.  model NULL: the model installed
+/* The candidate with the lowest predicted time (the shipped model was trained on
+ * stencils with a specialised kernel and no fields: it leaves other masks and
+ * CLOUDSIM to the heuristic).  model NULL: the model installed
  * with pskel_tuner_set_default_model, else the model shipped next to the
  * library (<libdir>/data/costmodel.bin, loaded on first use; the environment
  * variable PSKEL_TUNER_MODEL names another file, or "none"), else a fixed

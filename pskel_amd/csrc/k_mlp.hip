@@ -159,6 +159,7 @@ struct pskel_mlp {
     size_t np = 0;
     size_t off[kMaxLayers] = {0};  // parameter offset of layer l
     int device = 0;
+    bool shipped = false;       // the model beside the library, as its file holds it
     hipStream_t stream = nullptr;
     float* d_p = nullptr;       // parameters
     float* d_g = nullptr;       // gradients
@@ -244,6 +245,7 @@ hipError_t backward(pskel_mlp_t* m, int n, const float* x_std)
 namespace pskel {
 pskel_status_t mlp_predict_host(const pskel_mlp_t* mc, const float* x, size_t n, float* y);
 int mlp_inputs(const pskel_mlp_t* m) { return m ? m->sizes[0] : 0; }
+bool mlp_shipped(const pskel_mlp_t* m) { return m && m->shipped; }
 }
 
 extern "C" {
@@ -336,6 +338,7 @@ pskel_status_t pskel_mlp_get_params(const pskel_mlp_t* m, float* p, size_t n)
 pskel_status_t pskel_mlp_set_params(pskel_mlp_t* m, const float* p, size_t n)
 {
     if (!m || !p || n != m->np) return fail(PSKEL_ERR_INVALID_ARGUMENT, "parameter count");
+    m->shipped = false;
     PSKEL_HIP(hipSetDevice(m->device));
     PSKEL_HIP(hipMemcpy(m->d_p, p, n * sizeof(float), hipMemcpyHostToDevice));
     return PSKEL_OK;
@@ -347,6 +350,7 @@ pskel_status_t pskel_mlp_set_normalization(pskel_mlp_t* m, const float* mean, co
     if (!m || !mean || !sd || y_sd <= 0.f) return fail(PSKEL_ERR_INVALID_ARGUMENT, "bad normalisation");
     for (int i = 0; i < m->sizes[0]; ++i)
         if (!(sd[i] > 0.f)) return fail(PSKEL_ERR_INVALID_ARGUMENT, "feature std must be positive");
+    m->shipped = false;
     m->mean.assign(mean, mean + m->sizes[0]);
     m->sd.assign(sd, sd + m->sizes[0]);
     m->y_mean = y_mean;
@@ -398,6 +402,7 @@ pskel_status_t pskel_mlp_train(pskel_mlp_t* m, const float* x, const float* y, s
 {
     if (!m || !x || !y || n == 0 || epochs < 1 || batch < 1 || !(lr > 0.f))
         return fail(PSKEL_ERR_INVALID_ARGUMENT, "bad training arguments");
+    m->shipped = false;
     PSKEL_HIP(hipSetDevice(m->device));
     const int nin = m->sizes[0];
     const size_t bsz = std::min<size_t>((size_t)batch, n);
@@ -519,6 +524,7 @@ pskel_status_t pskel_mlp_load(const char* path, int32_t device, pskel_mlp_t** ou
              std::fread(&ym, 4, 1, f) == 1 && std::fread(&ys, 4, 1, f) == 1 && std::fread(p.data(), 4, p.size(), f) == p.size();
         if (ok) st = pskel_mlp_set_normalization(m, mean.data(), sd.data(), ym, ys);
         if (ok && st == PSKEL_OK) st = pskel_mlp_set_params(m, p.data(), p.size());
+        if (ok && st == PSKEL_OK) m->shipped = shipped_model_file(f);
     }
     std::fclose(f);
     if (!ok || st != PSKEL_OK) {

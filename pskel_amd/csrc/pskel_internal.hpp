@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cstddef>
 #include <cstdint>
+#include <cstdio>
 #include <cstring>
 #include <string>
 #include <thread>
@@ -285,6 +286,9 @@ bool ttile3d_shape_ok(const pskel_launch_cfg_t& cfg, int storage, int depth);
 
 // Deterministic second-stage reduction: out = sqrt(sum(partials[0..n))).
 hipError_t launch_reduce_partials(const double* partials, size_t n, double* out, hipStream_t st);
+
+// Is the open file the cost model shipped beside the library? (tuner.cpp)
+bool shipped_model_file(FILE* f);
 
 // Utilities.
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t st);

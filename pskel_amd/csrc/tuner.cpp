@@ -5,6 +5,7 @@
 // 1865-2076), which maximised an analytic objective without timing anything.
 #include <dlfcn.h>
 #include <hip/hip_runtime.h>
+#include <sys/stat.h>
 
 #include <algorithm>
 #include <cmath>
@@ -23,6 +24,7 @@ using namespace pskel;
 namespace pskel {
 pskel_status_t mlp_predict_host(const pskel_mlp_t* m, const float* x, size_t n, float* y);
 int mlp_inputs(const pskel_mlp_t* m);
+bool mlp_shipped(const pskel_mlp_t* m);
 }
 
 namespace {
@@ -34,7 +36,18 @@ std::once_flag g_model_once;
 // turns on any model.
 std::mutex g_predict_mutex;
 
-// The shipped cost model lives next to the library: <libdir>/data/costmodel.bin.
+// The shipped cost model lives next to the library: <libdir>/data/costmodel.bin
+// ("": the library's own path is unknown).
+std::string shipped_model_path()
+{
+    Dl_info info;
+    if (!dladdr((void*)&shipped_model_path, &info) || !info.dli_fname) return "";
+    std::string dir(info.dli_fname);
+    const size_t slash = dir.rfind('/');
+    dir = slash == std::string::npos ? std::string(".") : dir.substr(0, slash);
+    return dir + "/data/costmodel.bin";
+}
+
 // PSKEL_TUNER_MODEL names another model file, or "none" for no model (the
 // tuner then searches by measurement).
 void load_shipped_model()
@@ -44,12 +57,7 @@ void load_shipped_model()
         if (std::strcmp(env, "none") == 0 || env[0] == '\0') return;
         path = env;
     } else {
-        Dl_info info;
-        if (!dladdr((void*)&load_shipped_model, &info) || !info.dli_fname) return;
-        std::string dir(info.dli_fname);
-        const size_t slash = dir.rfind('/');
-        dir = slash == std::string::npos ? std::string(".") : dir.substr(0, slash);
-        path = dir + "/data/costmodel.bin";
+        path = shipped_model_path();
     }
     FILE* f = std::fopen(path.c_str(), "rb");
     if (!f) return;
@@ -62,6 +70,18 @@ void load_shipped_model()
     if (mlp_inputs(m) == PSKEL_TUNER_NFEAT) g_default_model = m;
     else pskel_mlp_destroy(m);
 }
+
+}  // namespace
+
+// Is the open file the shipped cost model?
+bool pskel::shipped_model_file(FILE* f)
+{
+    struct stat a, b;
+    return fstat(fileno(f), &a) == 0 && stat(shipped_model_path().c_str(), &b) == 0 && a.st_dev == b.st_dev &&
+           a.st_ino == b.st_ino;
+}
+
+namespace {
 
 pskel_launch_cfg_t tuned(int tx, int ty, int tz, int k)
 {
@@ -474,10 +494,10 @@ pskel_status_t pskel_tuner_choose(const pskel_mlp_t* model, const pskel_tune_que
         std::lock_guard<std::mutex> lock(g_predict_mutex);
         model = g_default_model;
     }
-    // the model's training queries hold no field stencils and no masks without a
-    // specialised kernel
+    // the shipped model's training queries hold no field stencils and no masks
+    // without a specialised kernel; any other model's may
     const int pat = classify(*d, q->ndim);
-    if (!model || pat == PAT_GENERIC || pat == PAT_CLOUD) {
+    if (!model || (mlp_shipped(model) && (pat == PAT_GENERIC || pat == PAT_CLOUD))) {
         *out = heuristic(*q, *d);
         return PSKEL_OK;
     }
