@@ -520,6 +520,30 @@ void spare_ring_copied(pskel::Grid& g, int radius)
     g.spare_width = radius;
 }
 
+// A run whose first launch, at the depth it names, would take a shape that is not
+// built is refused, though the tiles that run instead do not use the shape: the
+// LDS tile's rows (5-point and 3x3), CLOUDSIM's rows per lane and waves, and the
+// plain kernel's block where any mask runs on the LDS tile of k_points.hip.
+hipError_t named_launch(const pskel_grid_t* g, RunPlan plan, size_t iterations, int kmax, size_t every,
+                        const pskel_launch_cfg_t& cfg)
+{
+    if (plan.path == 3) {
+        const int64_t bx = cfg.block_x > 0 ? cfg.block_x : 64, by = cfg.block_y > 0 ? cfg.block_y : 4;
+        return bx * by > 1024 ? hipErrorInvalidConfiguration : hipSuccess;
+    }
+    if (!plan.rtile || plan.pattern == PAT_LIFE8) return hipSuccess;  // life rounds its rows
+    const int rows = cfg.tile_y;
+    if (plan.pattern == PAT_CLOUD) {
+        const bool ok = (rows <= 0 || rows == 1 || rows == 2 || rows == 4 || rows == 8) && cfg.tile_z <= 4;
+        return ok ? hipSuccess : hipErrorInvalidValue;
+    }
+    plan.rtile = false;
+    RtPlan q;
+    const bool fused = next_k(*g, plan, 0, iterations, kmax, every, &q) > 1;
+    const bool ok = cfg.tile_x != 0 || rows <= 0 || rows == 8 || rows == 16 || rows == 32 || rows == 64;
+    return fused && !ok ? hipErrorInvalidValue : hipSuccess;
+}
+
 // Issue all launches for `iterations` sweeps; advances the grid state.
 pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Points& pts, size_t iterations,
                      const pskel_launch_cfg_t& cfg, const RunPlan& plan, hipStream_t st,
@@ -528,6 +552,8 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
     const int ndim = g->ndim;
     const int kmax = (plan.path == 2) ? std::max(1, cfg.time_tile) : 1;
     const size_t every = cfg.residual_every > 0 ? (size_t)cfg.residual_every : 0;
+    if (const hipError_t e = named_launch(g, plan, iterations, kmax, every, cfg); e != hipSuccess)
+        return hip_fail(e, "stencil launch");
     size_t done = 0;
     int64_t nl = 0, nr = 0;
     while (done < iterations) {
