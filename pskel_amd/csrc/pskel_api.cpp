@@ -800,9 +800,15 @@ pskel_status_t plan_run(const pskel_grid_t* g, const pskel_stencil_desc_t* d, co
             fill_points(pts, *d, ndim);
             const size_t n = cells(g);
             const bool pays = ndim == 2 ? n >= 640 * 1024 : pts.np >= 8 || n >= 256 * 1024;
-            const bool tile = !pays ? false
-                              : ndim == 2 ? g->storage == PSKEL_DTYPE_F32 && points2d_ok((int)g->W, (int)g->H, pts)
-                                          : points3d_blocks(make_sweep3d(g, nullptr, nullptr, radius, nullptr), pts) > 0;
+            bool tile = false;
+            if (pays && ndim == 2) {
+                tile = g->storage == PSKEL_DTYPE_F32 && points2d_ok((int)g->W, (int)g->H, pts);
+            } else if (pays) {
+                // an allocation-free run's partials hold 65536 blocks: a thin grid may
+                // have more tiles than blocks of the plain kernel
+                const size_t nb = points3d_blocks(make_sweep3d(g, nullptr, nullptr, radius, nullptr), pts);
+                tile = nb > 0 && !(g->odd_2d_launches && cfg.residual_every > 0 && nb > kScratchPartials);
+            }
             if (tile) plan.path = 3;
         }
     }
