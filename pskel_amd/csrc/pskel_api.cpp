@@ -409,6 +409,7 @@ struct RunPlan {
     int pattern = PAT_GENERIC;
     int radius = 0;
     bool rtile = false;  // 2D fused sweeps on register tiles, as many per launch as pays
+    bool single = false; // single sweeps of a launch that names a fused tile
     // the run leaves the state one sweep before its result in the other buffer,
     // however deep its launches are (ends_single)
     bool keep_prev = false;
@@ -582,7 +583,7 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
         // a temporal run's leftover single sweeps use the tuned kernel's own
         // default tile (tile_y/tile_z describe the temporal tile there)
         pskel_launch_cfg_t one = cfg;
-        if (plan.path == 2 && k == 1) {
+        if ((plan.path == 2 || plan.single) && k == 1) {
             one.tile_y = 0;
             one.tile_z = 0;
             if (ndim == 3) {
@@ -767,7 +768,10 @@ pskel_status_t plan_run(const pskel_grid_t* g, const pskel_stencil_desc_t* d, co
         }
         // fused sweeps of the radius-1 f32 stencils run on register tiles, whatever
         // depth and tile the launch names
-        if (plan.pattern == PAT_LIFE8 && plan.path == 2 && !life_tiles_ok(g->pitch)) plan.path = 1;
+        if (plan.pattern == PAT_LIFE8 && plan.path == 2 && !life_tiles_ok(g->pitch)) {
+            plan.path = 1;
+            plan.single = true;
+        }
         if (plan.pattern == PAT_LIFE8 && plan.path == 2) plan.rtile = true;
         else plan.rtile = tunable && ndim == 2 && g->storage == PSKEL_DTYPE_F32 && cfg.time_tile > 1 && radius == 1 &&
                      rtile2d_ok(plan.pattern, (int)g->W, (int)g->H, g->pitch) &&
