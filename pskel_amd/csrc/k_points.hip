@@ -20,6 +20,8 @@
 // uniform branch per point keeps the loads from overlapping).  Measured, f32,
 // 3x3x3 weighted box with HALO faces: 192 x 225 x 260 32 us per sweep (3.5e11
 // cell-updates/s; plain 259 us), 256^3 40 us (400 us), 60 x 70 x 50 6.5 us (14 us).
+#include <cmath>
+
 #include "k_common.hpp"
 
 namespace pskel {
@@ -316,6 +318,40 @@ bool pt_kind(const Points& p)
 
 }  // namespace
 
+// The time of a sweep through the tile against the plain kernel's, whose block is bx
+// lanes along x by `by` along b.  Both are a launch and the larger of one block's (or
+// wave's) latency and the work: tiles stage and sum all their cells, those outside
+// the grid too; the plain kernel sums only the cells that take one (a copied face or
+// a ring costs it next to nothing), but lanes past a row's end cost it waves, and
+// points of HALO faces are checked one by one.  Microseconds, fitted to 1035 pairs
+// (31 3D grids from 40^3 to 256^3 and thin in each axis, 13 2D grids, 1 to 64
+// points, COPY and HALO, f32 and bf16): 1% behind the faster of the two on average,
+// where the tile throughout was 25% behind and up to 11 times slower (1 x 1500 x 1000
+// 27 points COPY, plain 4.3, tile 26; 5 x 200000 49 points 3.6 and 41).
+bool points_pay(const Points& p, bool is2d, int A, int B, int X, bool half, int bx, int by)
+{
+    PtPlan q;
+    if (!pt_kind(p) || !pt_plan(p, is2d, A, B, X, &q)) return false;
+    const bool halo = !is2d && p.boundary == PSKEL_BOUNDARY_HALO;
+    auto inner = [&](int n) { return (double)std::max(0, n - 2 * p.radius); };
+    const double cells = (double)A * B * X, sums = (is2d ? 1.0 : inner(A)) * inner(B) * inner(X), np = p.np;
+    if (!halo && sums == 0) return false;
+    const double waves = (double)((X + bx - 1) / bx) * ((B + by - 1) / by) * A * bx * by / kWave;
+    const double ms = sums / 1e6, mf = (cells - sums) / 1e6, mw = waves / 1e4;
+    const double plain = halo ? 0.85 + std::max(2.35 * mw + (1.0 * ms + 0.527 * mf) * np, 2.05 + 0.356 * np)
+                              : 1.81 + std::max(1.24 * mw + ms * (0.184 + 0.635 * np), 1.01 + 0.186 * np);
+    const double stage = (double)q.lds / sizeof(float) / 1e3;  // thousands of cells
+    const double per_cu = (double)((q.blocks + 255) / 256), at_once = (double)std::min<size_t>(4, (160 * 1024) / q.lds);
+    const double rounds = std::ceil(per_cu / at_once);
+    const double tile = halo ? 3.08 + std::max((0.0589 * np + 0.311 * stage) * rounds,
+                                               per_cu * (0.05 * np + 0.1525 * stage + (half ? 0.544 : 0.0)))
+                             : 4.04 + std::max((0.0715 * np + 0.227 * stage) * rounds,
+                                               per_cu * (0.0471 * np + 0.199 * stage + (half ? 0.047 : 0.0)));
+    // grids a cell or two thick (but along x) lie farthest from the fit
+    const bool thin = X >= 16 && cells < 0.25 * kPtCells * kPtThreads * (double)q.blocks;
+    return tile < (thin ? 0.75 : 0.95) * plain;
+}
+
 size_t points3d_blocks(const Sweep3D& s, const Points& p)
 {
     PtPlan q;
@@ -345,12 +381,6 @@ hipError_t launch_3d_points(const Sweep3D& s, const Points& p, int storage, hipS
     case PSKEL_DTYPE_F16: return pt_launch3d<PSKEL_DTYPE_F16>(q, p.kind, st);
     default: return hipErrorInvalidValue;
     }
-}
-
-bool points2d_ok(int W, int H, const Points& p)
-{
-    PtPlan q;
-    return pt_kind(p) && pt_plan(p, true, 1, H, W, &q);
 }
 
 hipError_t launch_2d_points_f32(const Sweep2D& s, const Points& p, hipStream_t st)

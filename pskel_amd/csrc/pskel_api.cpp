@@ -524,11 +524,11 @@ void spare_ring_copied(pskel::Grid& g, int radius)
 // A run whose first launch, at the depth it names, would take a shape that is not
 // built is refused, though the tiles that run instead do not use the shape: the
 // LDS tile's rows (5-point and 3x3), CLOUDSIM's rows per lane and waves, and the
-// plain kernel's block where any mask runs on the LDS tile of k_points.hip.
+// plain kernel's block where any mask runs (on the LDS tile of k_points.hip or not).
 hipError_t named_launch(const pskel_grid_t* g, RunPlan plan, size_t iterations, int kmax, size_t every,
                         const pskel_launch_cfg_t& cfg)
 {
-    if (plan.path == 3) {
+    if (plan.path == 3 || plan.path == 0) {
         const int64_t bx = cfg.block_x > 0 ? cfg.block_x : 64, by = cfg.block_y > 0 ? cfg.block_y : 4;
         return bx * by > 1024 ? hipErrorInvalidConfiguration : hipSuccess;
     }
@@ -793,25 +793,25 @@ pskel_status_t plan_run(const pskel_grid_t* g, const pskel_stencil_desc_t* d, co
             plan.path = 2;
         }
         if (!tunable) {
-            // no specialised kernel for this point set: the LDS tile of any
-            // mask, or the plain kernel where its halo does not fit and on
-            // small grids, whose few tiles leave the device idle.  Measured,
-            // plain / tile: 2D 512 x 512 3 points 3.5 / 4.8 us, 25 points 5.4 /
-            // 6.5; 800 x 1000 5.7 / 5.0 and 11.5 / 6.7; 3D 40^3 7 points 4.0 /
-            // 4.6, 13 points 7.0 / 5.4; 64^3 7 points 4.6 / 4.5
+            // no specialised kernel for this point set: the LDS tile of any mask
+            // where it is the faster one, else the plain kernel.  Small grids,
+            // whose few tiles leave the device idle, take the plain kernel.
+            // Measured, plain / tile: 2D 512 x 512 3 points 3.5 / 4.8 us, 25
+            // points 5.4 / 6.5; 800 x 1000 5.7 / 5.0 and 11.5 / 6.7
             plan.path = 0;
             Points pts;
             fill_points(pts, *d, ndim);
             const size_t n = cells(g);
-            const bool pays = ndim == 2 ? n >= 640 * 1024 : pts.np >= 8 || n >= 256 * 1024;
             bool tile = false;
-            if (pays && ndim == 2) {
-                tile = g->storage == PSKEL_DTYPE_F32 && points2d_ok((int)g->W, (int)g->H, pts);
-            } else if (pays) {
+            if (ndim == 2) {
+                tile = n >= 640 * 1024 && g->storage == PSKEL_DTYPE_F32 &&
+                       points_pay(pts, true, 1, (int)g->H, (int)g->W, false, bx, by);
+            } else if (pts.np >= 8 || n >= 256 * 1024) {
+                tile = points_pay(pts, false, (int)g->H, (int)g->W, (int)g->D, g->storage != PSKEL_DTYPE_F32, bx, by);
                 // an allocation-free run's partials hold 65536 blocks: a thin grid may
                 // have more tiles than blocks of the plain kernel
-                const size_t nb = points3d_blocks(make_sweep3d(g, nullptr, nullptr, radius, nullptr), pts);
-                tile = nb > 0 && !(g->odd_2d_launches && cfg.residual_every > 0 && nb > kScratchPartials);
+                if (tile && g->odd_2d_launches && cfg.residual_every > 0)
+                    tile = points3d_blocks(make_sweep3d(g, nullptr, nullptr, radius, nullptr), pts) <= kScratchPartials;
             }
             if (tile) plan.path = 3;
         }

@@ -254,8 +254,10 @@ size_t rtile2d_blocks(int W, int H, const RtPlan& q);
 hipError_t launch_2d_rtile(const Sweep2D& s, const Points& pts, const CloudArgs* cloud, int pattern, const RtPlan& q,
                            double* partials, hipStream_t st);
 
-// arbitrary masks through an LDS tile (k_points.hip): masks whose halo fits it
-bool points2d_ok(int W, int H, const Points& p);
+// arbitrary masks through an LDS tile (k_points.hip): its halo fits, and it is faster
+// than the plain kernel of block bx by `by` on a grid of extents (A, B, X) = (H, W, D)
+// in 3D, (1, H, W) in 2D (half: 16-bit storage)
+bool points_pay(const Points& p, bool is2d, int A, int B, int X, bool half, int bx, int by);
 hipError_t launch_2d_points_f32(const Sweep2D& s, const Points& p, hipStream_t st);
 hipError_t launch_3d_points(const Sweep3D& s, const Points& p, int storage, hipStream_t st);
 size_t points3d_blocks(const Sweep3D& s, const Points& p);  // 0: the halo does not fit

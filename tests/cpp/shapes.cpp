@@ -92,6 +92,61 @@ int shapes_ttile(const Job* j, int rows)
     return (int)launch_2d_ttile_f32(sweep(*j), points(*j), j->pattern, j->k, cfg, nullptr);
 }
 
+// one sweep of an arbitrary mask through its LDS tile: (H, W, D) in 3D, D = 1 and
+// pitched rows of W cells in 2D
+int shapes_points(const pskel_stencil_desc_t* d, int ndim, const void* src, void* dst, double* partials, int W, int H,
+                  int D, uint64_t pitch, int storage, float offset, int rounding, uint32_t seed, uint64_t sweep_no)
+{
+    Points p;
+    fill_points(p, *d, ndim);
+    if (ndim == 2) {
+        Sweep2D s;
+        s.src = src;
+        s.dst = dst;
+        s.ring_other = nullptr;
+        s.W = W;
+        s.H = H;
+        s.pitch = pitch;
+        s.radius = p.radius;
+        return (int)launch_2d_points_f32(s, p, nullptr);
+    }
+    Sweep3D s{};
+    s.src = src;
+    s.dst = dst;
+    s.W = W;
+    s.H = H;
+    s.D = D;
+    s.pitch = pitch;
+    s.radius = p.radius;
+    s.store_offset = offset;
+    s.partials = partials;
+    s.rounding = rounding;
+    s.seed = seed;
+    s.sweep = sweep_no;
+    s.c0 = storage == PSKEL_DTYPE_F32 ? 0.0f : scaled_sum_offset_term(p.coeff, p.np, offset);
+    return (int)launch_3d_points(s, p, storage, nullptr);
+}
+
+// its blocks (0: the halo does not fit) and whether a run takes it over the plain
+// kernel with blocks of bx by `by` lanes
+uint64_t shapes_points_blocks(const pskel_stencil_desc_t* d, int W, int H, int D)
+{
+    Points p;
+    fill_points(p, *d, 3);
+    Sweep3D s{};
+    s.W = W;
+    s.H = H;
+    s.D = D;
+    return points3d_blocks(s, p);
+}
+
+int shapes_points_pay(const pskel_stencil_desc_t* d, int ndim, int W, int H, int D, int half, int bx, int by)
+{
+    Points p;
+    fill_points(p, *d, ndim);
+    return ndim == 2 ? points_pay(p, true, 1, H, W, half != 0, bx, by) : points_pay(p, false, H, W, D, half != 0, bx, by);
+}
+
 // the next launch of a run with `rem` sweeps to go: {r, nw, k}
 void shapes_plan(int pattern, int W, int H, uint64_t rem, int odd, int32_t* out)
 {

@@ -16,7 +16,9 @@ class Job(C.Structure):
 def lib():
     l = C.CDLL(dropin.driver("libshapes.so"))
     assert l.shapes_job_size() == C.sizeof(Job)
-    l.shapes_rtile_blocks.restype = C.c_uint64
+    l.shapes_rtile_blocks.restype = l.shapes_points_blocks.restype = C.c_uint64
+    l.shapes_points.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int,
+                                C.c_uint64, C.c_int, C.c_float, C.c_int, C.c_uint32, C.c_uint64]
     l.shapes_plan.argtypes = [C.c_int, C.c_int, C.c_int, C.c_uint64, C.c_int, C.POINTER(C.c_int32)]
     return l
 
