@@ -113,7 +113,8 @@ typedef struct pskel_launch_cfg {
                                run fuse as many sweeps per launch as pay on register tiles;
                                the tiles below hold where those do not run (mask range above 1,
                                grids up to 8 cells wide or over 2 GiB, the 9-point stencil
-                               above 12M cells).
+                               above 12M cells, tall grids narrower than a register tile
+                               and runs of 2 or 3 sweeps where they are slower).
                                2D: k <= 4 (8 for life): tile (0, CY, 0) LDS tiles of CY in
                                {8,16,32,64} rows (0: 32), or tile (4, 0, S) the register march,
                                S rows per segment (0: automatic; grids wider than 8 cells);

@@ -692,10 +692,37 @@ bool cloud_fields_fit(const pskel_grid_t* g)
     return true;
 }
 
+// Do the register tiles (256 columns) beat the kernels a 2D f32 launch names?  They
+// lose on tall grids narrower than a tile, whose idle lanes cost as much as busy
+// ones once the blocks fill the device, and in runs of two or three sweeps, where
+// the halo is not paid back.  Measured, us, named / tiles:
+//   9-point, LDS tiles (120 columns) of 16 rows: 20000 x 40, 40 sweeps 103 / 169,
+//   100000 x 100 414 / 616; of 32 rows: 20000 x 40, 3 sweeps 12.2 / 18.4; from 420
+//   blocks on (312: level), and 40000 x 270, three columns of those against two of
+//   these, 463 / 540;
+//   5-point, LDS tiles of 16 rows, 3 sweeps: 20000 x 9 1.14 times slower;
+//   9-point, register march, 2 and 3 sweeps: 2048^2 1.15 and 1.03 times slower,
+//   3000^2 1.18 and 1.12, 40000 x 300 1.16 and 1.13 (under 3M cells level or faster);
+//   CLOUDSIM, single sweeps: 9000 x 100, 3 sweeps 1.29 times slower, 100000 x 40
+//   67 / 137, 7 sweeps 154 / 219; 20000 x 40, 7 sweeps level, 40 1.16 times faster.
+// A residual step is reduced in the tiles' launch: there they win (0.4 to 0.85).
+bool rtile_pays(int pattern, const pskel_grid_t* g, const pskel_launch_cfg_t& cfg, size_t iterations)
+{
+    const size_t W = g->W, H = g->H, every = cfg.residual_every > 0 ? (size_t)cfg.residual_every : 0;
+    const size_t run = every ? std::min(iterations, every) : iterations;  // sweeps that may share a launch
+    if (pattern == PAT_CLOUD) return !((W <= 256 && H > 6000 && run <= 3) || (W <= 100 && H > 25000 && run < 8));
+    if (every && every <= iterations) return true;
+    if (cfg.tile_x != 0) return !(pattern == PAT_BOX9 && run <= 3 && (W * H >= 3000000 || H >= 20000));
+    const size_t rows = cfg.tile_y > 0 ? (size_t)cfg.tile_y : 32;
+    if (pattern == PAT_BOX9 && W > 240 && W <= 360 && H >= 20000) return false;
+    if (W > 120 || H <= 420 * rows) return true;
+    return pattern == PAT_J5 && (run > 3 || W > 64 || rows > 16);
+}
+
 // Validate a run and choose its kernels (shared by the resident runner and the
 // host-staged pipeline).
 pskel_status_t plan_run(const pskel_grid_t* g, const pskel_stencil_desc_t* d, const pskel_launch_cfg_t& cfg,
-                        RunPlan& plan)
+                        size_t iterations, RunPlan& plan)
 {
     const int ndim = g->ndim;
     if (d->npoints < 1 || d->npoints > PSKEL_MAX_POINTS)
@@ -766,8 +793,8 @@ pskel_status_t plan_run(const pskel_grid_t* g, const pskel_stencil_desc_t* d, co
                 if (radius != 1) return fail(PSKEL_ERR_UNSUPPORTED, "2D register march: mask range 1");
             }
         }
-        // fused sweeps of the radius-1 f32 stencils run on register tiles, whatever
-        // depth and tile the launch names
+        // fused sweeps of the radius-1 f32 stencils run on register tiles where those
+        // are faster, whatever depth and tile the launch names
         if (plan.pattern == PAT_LIFE8 && plan.path == 2 && !life_tiles_ok(g->pitch)) {
             plan.path = 1;
             plan.single = true;
@@ -775,6 +802,7 @@ pskel_status_t plan_run(const pskel_grid_t* g, const pskel_stencil_desc_t* d, co
         if (plan.pattern == PAT_LIFE8 && plan.path == 2) plan.rtile = true;
         else plan.rtile = tunable && ndim == 2 && g->storage == PSKEL_DTYPE_F32 && cfg.time_tile > 1 && radius == 1 &&
                      rtile2d_ok(plan.pattern, (int)g->W, (int)g->H, g->pitch) &&
+                     rtile_pays(plan.pattern, g, cfg, iterations) &&
                      (plan.pattern != PAT_CLOUD || cloud_fields_fit(g));
         // the allocation-free run's partials hold 65536 blocks
         if (plan.rtile && g->odd_2d_launches && rtile2d_partials(*g, plan, cfg) > kScratchPartials) plan.rtile = false;
@@ -863,7 +891,7 @@ pskel_status_t pskel::run_async(pskel_grid_t* g, const pskel_stencil_desc_t* d, 
     *launches = 0;
     if (cfg.residual_every > 0 || cfg.use_graph) return fail(PSKEL_ERR_UNSUPPORTED, "residuals or graphs here");
     RunPlan plan;
-    pskel_status_t st = plan_run(g, d, cfg, plan);
+    pskel_status_t st = plan_run(g, d, cfg, iterations, plan);
     if (st != PSKEL_OK) return st;
     if (iterations == 0) return PSKEL_OK;
     if ((plan.path == 2 || plan.rtile) && g->ndim == 2 && !g->buf[2]) return fail(PSKEL_ERR_RUNTIME, "spare buffer missing");
@@ -1151,7 +1179,7 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
     }
     // ---- validation -------------------------------------------------------
     RunPlan plan;
-    if ((st = plan_run(g, d, cfg, plan)) != PSKEL_OK) return st;
+    if ((st = plan_run(g, d, cfg, iterations, plan)) != PSKEL_OK) return st;
     const int ndim = g->ndim;
     const int radius = plan.radius;
     if (stats) stats->sweeps = (int64_t)iterations;
@@ -1383,7 +1411,7 @@ extern "C" pskel_status_t pskel_run_iterative_noalloc(const pskel_grid_desc_t* d
     g.buf[1] = out;
     g.odd_2d_launches = true;
     RunPlan plan;
-    pskel_status_t st = plan_run(&g, d, cfg, plan);
+    pskel_status_t st = plan_run(&g, d, cfg, iterations, plan);
     if (st != PSKEL_OK) return st;
     Points pts;
     fill_points(pts, *d, g.ndim);
