@@ -280,7 +280,7 @@ hipError_t stage_copy(pskel_grid_t* g, void* dbuf, void* stage, size_t r0, size_
 {
     const size_t rb = row_cells(g) * g->elem, pb = g->pitch * g->elem;
     char* dev = (char*)dbuf + r0 * pb;
-    if (pb != rb && g->bounce) {
+    if (pb != rb && n > 1 && g->bounce) {  // (one row is one copy as it is)
         if (kind == hipMemcpyHostToDevice) {
             const hipError_t e = hipMemcpyAsync(g->bounce, stage, n * rb, kind, g->stream);
             return e == hipSuccess ? launch_rows(dev, pb, g->bounce, rb, rb, n, g->stream) : e;
