@@ -353,7 +353,9 @@ pskel_status_t pskel_grid_set_field(pskel_grid_t* grid, int32_t slot, pskel_fiel
  *      fuses per launch: 1 (or 0) or 3 for F32, 1, 3, 5 or 7 for life (mask
  *      range 1).  Above 1, life and F32 at mask range 1 run on tiles held in
  *      registers, at the depth that suits the batch and the run's length; F32
- *      at a wider range runs LDS tiles of tile_y rows (16 or 32; default 16).
+ *      at a wider range, and where they are faster (few or narrow 3x3 grids,
+ *      short runs of both stencils together), runs LDS tiles of tile_y rows
+ *      (16 or 32; default 16) at depth 3.
  *      A launch fuses an odd number k, so it moves a grid's state to its other
  *      buffer: N sweeps run as N / k launches of k and the rest as one odd
  *      launch or two (r - 1, then 1); a grid whose launches of k = time_tile

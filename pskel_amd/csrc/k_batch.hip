@@ -12,8 +12,8 @@
 // with the other families' (no grid belongs to two).
 //
 // Temporal depth.  Each grid fuses K sweeps per launch (K odd: 1 or 3 for the
-// f32 stencils, on register tiles (k_rtile2d.hpp) or, where those do not run,
-// the LDS temporal tile; 1, 3, 5 or 7 for life, on bit-packed tiles
+// f32 stencils, on register tiles (k_rtile2d.hpp) or, where those do not run
+// or are slower, the LDS temporal tile; 1, 3, 5 or 7 for life, on bit-packed tiles
 // (k_ltile.hpp); K = 1 runs the one-sweep tiles of k_tiles2d.hpp).  A grid of
 // a family that holds its tiles in registers (bit-packed life, the f32 register
 // tiles) fuses as many sweeps as pay for the whole family, at least the depths
@@ -51,7 +51,7 @@ struct BatchEntry {
     int radius;
     int kind;
     int ry;           // K = 1: rows per lane; LDS tiles: tile rows
-    int rtile;        // f32 at K = 3 on register tiles
+    int rtile;        // f32 at K = 3 on register tiles (choose_f32_tiles)
     int depth;        // K, sweeps fused per launch (odd); of a tile family: the tiles' halo
     int full;         // launches of K sweeps
     int tail0, tail1, tail2;  // sweeps of the launches after them (odd; 0: none)
@@ -214,6 +214,14 @@ void tile_grid(BatchEntry& e, int K)
     e.ntiles = e.tiles_x * rt_tiles(e.H, kBatchTileH, K);
 }
 
+// LDS tiles of a grid: 3 sweeps, e.ry rows
+void lds_grid(BatchEntry& e)
+{
+    e.depth = kTTileK;
+    e.tiles_x = (e.W + kTTileCX - 1) / kTTileCX;
+    e.ntiles = e.tiles_x * ((e.H + e.ry - 1) / e.ry);
+}
+
 int launches_of(const BatchEntry& e) { return e.full + (e.tail0 > 0) + (e.tail1 > 0) + (e.tail2 > 0); }
 
 }  // namespace
@@ -225,6 +233,9 @@ struct pskel_batch {
     int* d_items = nullptr;          // the work items of each family, one list after the other
     size_t items_cap = 0;
     std::vector<int> asked;          // depth asked for each grid
+    // f32 grids that fit the register tiles and the LDS tiles: 1 LDS tiles named, 2 the
+    // register march (0: others)
+    std::vector<char> either;
     int fam_slots[BF_COUNT] = {};    // blocks of a family's kernel the device holds at once
     int fam_items[BF_COUNT] = {};    // items per family
     int fam_first[BF_COUNT] = {};    // offset of a family's list in d_items
@@ -311,11 +322,52 @@ int family_depth(const pskel_batch_t* b, int f, size_t n)
     return best;
 }
 
+// Register or LDS tiles for the f32 grids that fit both, for runs of n sweeps.  Where
+// the launch names LDS tiles: the 3x3 stencil's 64-row register tiles take 2 us a sweep however few
+// there are, so they need about one for every second CU (a 700 x 900 grid, 52 tiles,
+// 12 sweeps: LDS 37 us, register 48; 24 grids, 325 tiles: 0.87 times the LDS time),
+// and grids up to 120 wide leave half their lanes idle (4 grids of 20000 x 30, 105
+// sweeps 1197 and 1533; a few among wider ones ride along).  And the LDS tiles run
+// both stencils in one kernel: a kernel more costs a run about 20 us, the graph's fork
+// and join (4 to 48 mixed grids, 3 sweeps, 2.2 to 2.4 times the LDS time), which the
+// register tiles win back at 0.3 (5-point) and 0.5 us (3x3) per million cells and sweep.
+void choose_f32_tiles(pskel_batch_t* b, size_t n)
+{
+    double mj = 0.0, mb = 0.0, narrow = 0.0;  // million cells
+    int64_t box_tiles = 0;
+    bool march = false;
+    for (size_t i = 0; i < b->host_tab.size(); ++i) {
+        if (!b->either[i]) continue;
+        BatchEntry t = b->host_tab[i];
+        tile_grid(t, kTTileK);
+        const double m = 1e-6 * t.W * t.H;
+        if (t.kind == BK_J5) {
+            mj += m;
+        } else {
+            mb += m;
+            if (t.W <= kTTileCX) narrow += m;
+            box_tiles += t.ntiles;
+            march |= b->either[i] == 2;
+        }
+    }
+    bool box = march || (box_tiles >= (n < 20 ? 200 : 130) && narrow < 0.5 * mb), j5 = true;
+    if (mj > 0.0 && mb > 0.0 && (0.3 * mj + (box ? 0.5 * mb : 0.0)) * (double)n <= 20.0) box = j5 = false;
+    for (size_t i = 0; i < b->host_tab.size(); ++i) {
+        if (!b->either[i]) continue;
+        BatchEntry& e = b->host_tab[i];
+        e.rtile = e.kind == BK_J5 ? j5 : box;
+        if (e.rtile) tile_grid(e, kTTileK);
+        else lds_grid(e);
+    }
+}
+
 // Depths, schedules and item order for `n` sweeps: in each family's list, grids
 // with more launches first.
 pskel_status_t plan_batch(pskel_batch_t* b, size_t n)
 {
     const size_t ng = b->host_tab.size();
+    choose_f32_tiles(b, n);
+    count_items(b);
     for (int f = BF_BITS; f < BF_COUNT; ++f) {
         if (b->fam_items[f] == 0) continue;
         const int K = family_depth(b, f, n);
@@ -422,6 +474,7 @@ pskel_status_t pskel_batch_create(pskel_grid_t* const* grids, const pskel_stenci
         const pskel_stencil_desc_t& d = descs[i];
         const int pat = classify(d, 2);
         BatchEntry e{};
+        char either = 0;
         if (pat == PAT_J5 && g->storage == PSKEL_DTYPE_F32) e.kind = BK_J5;
         else if (pat == PAT_BOX9 && g->storage == PSKEL_DTYPE_F32) e.kind = BK_BOX9;
         else if (pat == PAT_LIFE8 && g->storage == PSKEL_DTYPE_U8) e.kind = BK_LIFE;
@@ -458,9 +511,9 @@ pskel_status_t pskel_batch_create(pskel_grid_t* const* grids, const pskel_stenci
                 e.ntiles = e.tiles_x * ((e.H + kBatchWaves * 4 - 1) / (kBatchWaves * 4));
             }
         } else {
-            // 3 sweeps per launch: the register tiles, whatever tile the launch
-            // names; LDS tiles of 120 columns and 16 or 32 rows at a mask range
-            // above 1 and on grids the register tiles do not take
+            // 3 sweeps per launch: the register tiles; LDS tiles of 120 columns and
+            // 16 or 32 rows at a mask range above 1, on grids the register tiles do
+            // not take and where they are faster (choose_f32_tiles)
             const bool march = cfgs && cfgs[i].tile_x == kMarch2DVd;
             if (march) {
                 if (depth != 3) return reject(PSKEL_ERR_UNSUPPORTED, "the batched register march runs 3 sweeps per launch");
@@ -472,15 +525,16 @@ pskel_status_t pskel_batch_create(pskel_grid_t* const* grids, const pskel_stenci
             if (depth != kTTileK) return reject(PSKEL_ERR_UNSUPPORTED, "batched f32 depths are 1 or 3");
             const int cy = cfgs && cfgs[i].tile_y > 0 && !march ? cfgs[i].tile_y : 16;
             if (cy != 16 && cy != 32) return reject(PSKEL_ERR_UNSUPPORTED, "batched f32 temporal tiles have 16 or 32 rows");
+            e.ry = cy;
             if (radius == 1 && rt_fits(e.W, e.H, g->pitch)) {
                 e.rtile = 1;
                 tile_grid(e, depth);
+                either = march ? 2 : 1;
             } else {
-                e.ry = cy;
-                e.tiles_x = (e.W + kTTileCX - 1) / kTTileCX;
-                e.ntiles = e.tiles_x * ((e.H + cy - 1) / cy);
+                lds_grid(e);
             }
         }
+        b->either.push_back(either);
         b->grids.push_back(g);
         b->host_tab.push_back(e);
         b->asked.push_back(depth);
