@@ -123,9 +123,10 @@ struct FamLds<BF_J5> : RtLds<kBatchTileRows, kBatchTileWaves> {};
 template <>
 struct FamLds<BF_BOX9> : RtLds<kBatchTileRows, kBatchTileWaves> {};
 
+// (the life tiles fit 64 registers, four blocks per CU)
 template <int FAM>
-__global__ __launch_bounds__(fam_waves(FAM) * kWave) void k_batch(const BatchEntry* __restrict__ tab, const int* __restrict__ item_grid,
-                                               int nitems, int launch)
+__global__ __launch_bounds__(fam_waves(FAM) * kWave, FAM == BF_BITS ? 8 : 1) void k_batch(
+    const BatchEntry* __restrict__ tab, const int* __restrict__ item_grid, int nitems, int launch)
 {
     __shared__ FamLds<FAM> L;
     const int parity = launch & 1;
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(fam_waves(FAM) * kWave) void k_batch(const BatchEnt
             const int lane = (int)threadIdx.x, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
             const int tx = t % E.tiles_x, ty = t / E.tiles_x;
             if constexpr (FAM == BF_BITS) {
-                life_tile(s, tx, ty, E.depth, k, lane, wave, L);
+                life_tile<kBatchTileRows, kBatchTileWaves, false>(s, tx, ty, E.depth, k, lane, wave, L);
             } else {
                 RtParams p;
                 p.coeff = E.coeff;

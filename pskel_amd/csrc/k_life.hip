@@ -85,7 +85,10 @@ hipError_t launch_life_tiles(const Sweep2D& s, const RtPlan& q, hipStream_t st)
     const int ntx = lt_tiles(s.W, kLtCols, 32);
     const dim3 grid((unsigned)(ntx * lt_tiles(s.H, q.r * q.nw, q.k))), block(q.nw * kWave);
 #define PSKEL_LT(R, NW) \
-    if (q.r == R && q.nw == NW) hipLaunchKernelGGL((k_life_tiles<R, NW>), grid, block, 0, st, s, ntx, q.k)
+    if (q.r == R && q.nw == NW && s.prev)                                                     \
+        hipLaunchKernelGGL((k_life_tiles<R, NW, true>), grid, block, 0, st, s, ntx, q.k);     \
+    else if (q.r == R && q.nw == NW)                                                          \
+        hipLaunchKernelGGL((k_life_tiles<R, NW, false>), grid, block, 0, st, s, ntx, q.k)
     // the shapes of kLtShapes
     PSKEL_LT(2, 8);
     else PSKEL_LT(2, 16);

@@ -121,8 +121,9 @@ __device__ __forceinline__ void lt_sums(uint32_t x, uint32_t& h0, uint32_t& h1, 
 }
 
 // Tile (tx, ty) of a board tiled for K generations, by the block's NW waves; k
-// run (1 <= k <= K).  Every wave must call it (it synchronises the block).
-template <int R, int NW>
+// run (1 <= k <= K).  Every wave must call it (it synchronises the block).  With KEEP
+// the state before the last generation goes to s.prev, if set.
+template <int R, int NW, bool KEEP>
 __device__ __forceinline__ void life_tile(const Sweep2D& s, int tx, int ty, int K, int k, int lane, int wave,
                                           LtLds<R, NW>& L)
 {
@@ -200,6 +201,48 @@ __device__ __forceinline__ void life_tile(const Sweep2D& s, int tx, int ty, int 
     // rows [cy0 - left, cy1 + left) are needed once `left` generations remain
     auto needed = [&](int left) { return wy < cy1 + left && wy + R > cy0 - left && wy < H; };
 
+    // the tile's own interior rows (with `ring` the ring's too); a lane holding a ring
+    // column writes the ring value it holds, which is dst's own.  The padding of a row may be the caller's:
+    // a 16-byte half that reaches past W is stored in pieces of 8, 4, 2 and 1 cells.
+    auto store = [&](void* to, bool ring) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rd = plane_rsrc((uint8_t*)to + (size_t)y0 * pitch, bytes);
+        // recomputed from the lane: hoisted above the generations, these would hold
+        // registers there
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int xl = x0 + ln * 32;
+        const int cells = xl >= cx0 && xl < cx1 ? min(W - xl, 32) : 0;  // this lane's cells on the board
+        const bool ragged = W % 16 != 0 && x0 + kLtCols >= W;           // uniform
+        const int part = ragged ? cells & 15 : 0;                       // cells of such a half
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int y = wy + i;
+            if (y < cy0 || y >= cy1 || (!ring && (y < 1 || y > H - 2))) continue;  // uniform
+            u32x4_t a, b;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                a[q] = lt_unpack(c[i], q);
+                b[q] = lt_unpack(c[i], q + 4);
+            }
+            const uint32_t o = (uint32_t)(wave * R + i) * p + (uint32_t)xl;
+            __builtin_amdgcn_raw_buffer_store_b128(a, rd, (int)(cells >= 16 ? o : kNoAccess), 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(b, rd, (int)(cells == 32 ? o + 16 : kNoAccess), 0, 0);
+            if (!ragged) continue;
+            const uint32_t h = o + (cells & 16);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[q] = cells & 16 ? b[q] : a[q];
+            const u32x2_t two = {a[0], a[1]};
+            __builtin_amdgcn_raw_buffer_store_b64(two, rd, (int)(part & 8 ? h : kNoAccess), 0, 0);
+            const uint32_t w4 = part & 8 ? a[2] : a[0];
+            __builtin_amdgcn_raw_buffer_store_b32(w4, rd, (int)(part & 4 ? h + (part & 8) : kNoAccess), 0, 0);
+            const uint32_t w2 = part & 8 ? (part & 4 ? a[3] : a[2]) : (part & 4 ? a[1] : a[0]);
+            __builtin_amdgcn_raw_buffer_store_b16((uint16_t)w2, rd, (int)(part & 2 ? h + (part & 12) : kNoAccess), 0,
+                                                  0);
+            __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(part & 2 ? w2 >> 16 : w2), rd,
+                                                 (int)(part & 1 ? h + (part & 14) : kNoAccess), 0, 0);
+        }
+    };
+
     int l = 0;
 #pragma unroll 1
     for (; l < k; ++l) {
@@ -209,6 +252,9 @@ __device__ __forceinline__ void life_tile(const Sweep2D& s, int tx, int ty, int 
         const bool act = needed(k - 1 - l);
         __syncthreads();
         if (!act) break;
+        // uniform; an even k's goes to the buffer that holds its ring, an odd one's (at
+        // least 3) to one that does not
+        if (KEEP && l + 1 == k && s.prev) store(s.prev, k & 1);
         uint32_t hp0, hp1, hc0, hc1, mc0, mc1, m0, m1;
         lt_sums(x[up][1][lane], hp0, hp1, m0, m1);
         lt_sums(c[0], hc0, hc1, mc0, mc1);
@@ -244,50 +290,17 @@ __device__ __forceinline__ void life_tile(const Sweep2D& s, int tx, int ty, int 
         return;
     }
 
-    // the tile's own interior rows; a lane holding a ring column writes the ring
-    // value it holds, which is dst's own.  The padding of a row may be the caller's:
-    // a 16-byte half that reaches past W is stored in pieces of 8, 4, 2 and 1 cells.
-    const __amdgpu_buffer_rsrc_t rd = plane_rsrc((uint8_t*)s.dst + (size_t)y0 * pitch, bytes);
-    const bool own = xs >= cx0 && xs < cx1;
-    const int cells = own ? min(W - xs, 32) : 0;          // this lane's cells on the board
-    const bool ragged = W % 16 != 0 && x0 + kLtCols >= W;  // uniform
-    const int part = ragged ? cells & 15 : 0;              // cells of such a half
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-        const int y = wy + i;
-        if (y < cy0 || y >= cy1 || y < 1 || y > H - 2) continue;  // uniform
-        u32x4_t a, b;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            a[q] = lt_unpack(c[i], q);
-            b[q] = lt_unpack(c[i], q + 4);
-        }
-        const uint32_t o = off(i);
-        __builtin_amdgcn_raw_buffer_store_b128(a, rd, (int)(cells >= 16 ? o : kNoAccess), 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(b, rd, (int)(cells == 32 ? o + 16 : kNoAccess), 0, 0);
-        if (!ragged) continue;
-        const uint32_t h = o + (cells & 16);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) a[q] = cells & 16 ? b[q] : a[q];
-        const u32x2_t two = {a[0], a[1]};
-        __builtin_amdgcn_raw_buffer_store_b64(two, rd, (int)(part & 8 ? h : kNoAccess), 0, 0);
-        const uint32_t w4 = part & 8 ? a[2] : a[0];
-        __builtin_amdgcn_raw_buffer_store_b32(w4, rd, (int)(part & 4 ? h + (part & 8) : kNoAccess), 0, 0);
-        const uint32_t w2 = part & 8 ? (part & 4 ? a[3] : a[2]) : (part & 4 ? a[1] : a[0]);
-        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)w2, rd, (int)(part & 2 ? h + (part & 12) : kNoAccess), 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(part & 2 ? w2 >> 16 : w2), rd,
-                                             (int)(part & 1 ? h + (part & 14) : kNoAccess), 0, 0);
-    }
+    store(s.dst, false);
 }
 
-template <int R, int NW>
+template <int R, int NW, bool KEEP>
 __global__ __launch_bounds__(NW * kWave, 8) void k_life_tiles(Sweep2D s, int ntx, int K)
 {
     __shared__ LtLds<R, NW> L;
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int t = (int)xcd_remap(blockIdx.x, gridDim.x);
-    life_tile<R, NW>(s, t % ntx, t / ntx, K, K, lane, wave, L);
+    life_tile<R, NW, KEEP>(s, t % ntx, t / ntx, K, K, lane, wave, L);
 }
 
 }  // namespace

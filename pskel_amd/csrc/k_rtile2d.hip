@@ -63,16 +63,9 @@ hipError_t rt_go(const Sweep2D& s, const RtParams& p, int k, double* partials, h
 {
     const int ntx = rt_tiles(s.W, kRtCols, rt_halo_cols(k)), nty = rt_tiles(s.H, R * NW, k);
     const dim3 grid((unsigned)(ntx * nty)), block(NW * kWave);
-    if (partials) {
-        hipLaunchKernelGGL((k2d_rtile<PAT, R, NW, true, true>), grid, block, 0, st, s, p, ntx, k, partials);
-        return hipGetLastError();
-    }
-    if (s.prev) {
-        if constexpr (PAT != PAT_CLOUD) return hipErrorInvalidValue;
-        else hipLaunchKernelGGL((k2d_rtile<PAT, R, NW, false, true>), grid, block, 0, st, s, p, ntx, k, partials);
-        return hipGetLastError();
-    }
-    hipLaunchKernelGGL((k2d_rtile<PAT, R, NW, false, false>), grid, block, 0, st, s, p, ntx, k, partials);
+    if (partials) hipLaunchKernelGGL((k2d_rtile<PAT, R, NW, true, true>), grid, block, 0, st, s, p, ntx, k, partials);
+    else if (s.prev) hipLaunchKernelGGL((k2d_rtile<PAT, R, NW, false, true>), grid, block, 0, st, s, p, ntx, k, partials);
+    else hipLaunchKernelGGL((k2d_rtile<PAT, R, NW, false, false>), grid, block, 0, st, s, p, ntx, k, partials);
     return hipGetLastError();
 }
 

@@ -175,9 +175,9 @@ __device__ __forceinline__ void rt_row(const RtParams& p, const float (&u)[4], c
 // Tile (tx, ty) of a grid tiled for K sweeps, by the block's NW waves; k sweeps
 // run (1 <= k <= K).  Every wave must call it (it synchronises the block).
 // With RES returns this lane's sum of squared changes of the last sweep over the
-// tile's own cells, ring cells included.  With KEEP an even k also stores the state
-// before its last sweep in s.prev, if set (in the loop of every kernel the check
-// would cost the 5-point 8-row tiles a wave per SIMD).
+// tile's own cells, ring cells included.  With KEEP the state before the last sweep
+// goes to s.prev, if set (in the loop of every kernel the check would cost the 5-point
+// 8-row tiles a wave per SIMD).
 template <int PAT, int R, int NW, bool RES, bool KEEP>
 __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, int tx, int ty, int K, int k, int lane,
                                           int wave, RtLds<R, NW>& L)
@@ -341,11 +341,11 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
 
     const __amdgpu_buffer_rsrc_t rd = plane_rsrc(s.dst, bytes);
     const bool own_x = xs >= cx0 && xs < cx1;
-    // the tile's own interior rows; a lane vector holding a ring column writes
+    // the tile's own interior rows (with `ring` the ring's too); a lane vector holding a ring column writes
     // the ring value it holds, which is dst's own.  The padding of a row may be
     // the caller's (not CLOUDSIM's, whose buffers are a grid's): the vector that
     // reaches past W stores its cells as a pair and a single.
-    auto store = [&](const __amdgpu_buffer_rsrc_t& r, auto off_t) __attribute__((always_inline)) {
+    auto store = [&](const __amdgpu_buffer_rsrc_t& r, auto off_t, bool ring) __attribute__((always_inline)) {
         // 5-point and 9-point: recomputed from the lane; hoisted above the sweeps,
         // these would hold registers there (5-point 8-row tiles 81 for 72, two waves
         // per SIMD less)
@@ -362,7 +362,7 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
 #pragma unroll
         for (int i = 0; i < R; ++i) {
             const int y = wy + i;
-            if (y < cy0 || y >= cy1 || y < 1 || y > H - 2) continue;  // uniform
+            if (y < cy0 || y >= cy1 || (!ring && (y < 1 || y > H - 2))) continue;  // uniform
             const uint32_t o = (uint32_t)y * pb + (uint32_t)x * 4u;
             u32x4_t v;
 #pragma unroll
@@ -394,13 +394,14 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
     constexpr std::integral_constant<int, 0> at0;
     constexpr std::integral_constant<int, 1> at1;
     auto finish = [&](auto off_t) __attribute__((always_inline)) {
-        store(rd, off_t);
+        store(rd, off_t, false);
         return rr;
     };
-    // before the last of an even number of sweeps
-    auto keep_prev = [&]() __attribute__((always_inline)) {
+    // before the last sweep: of an even number to the buffer that holds its ring, of an
+    // odd one (at least 3) to one that does not
+    auto keep_prev = [&](auto off_t) __attribute__((always_inline)) {
         if (!KEEP || !s.prev) return;  // uniform
-        store(plane_rsrc(s.prev, bytes), at0);
+        store(plane_rsrc(s.prev, bytes), off_t, decltype(off_t)::value == 1);
     };
     int l = 0;
     // with RES the last sweep is another copy of the code: its sums, and the
@@ -409,18 +410,20 @@ __device__ __forceinline__ double rt_tile(const Sweep2D& s, const RtParams& p, i
     for (;;) {
         if (!exchange(l, L.x[0], a[1], a[R])) return rr;
         if (RES && l + 1 == k) {
+            keep_prev(at1);
             sweep(at1, true, std::bool_constant<RES>());
             return finish(at0);
         }
+        if (KEEP && l + 1 == k) keep_prev(at1);
         sweep(at1, true, std::false_type());
         if (++l == k) return finish(at0);
         if (!exchange(l, L.x[1], a[0], a[R - 1])) return rr;
         if (RES && l + 1 == k) {
-            keep_prev();
+            keep_prev(at0);
             sweep(at0, false, std::bool_constant<RES>());
             return finish(at1);
         }
-        if (KEEP && l + 1 == k) keep_prev();
+        if (KEEP && l + 1 == k) keep_prev(at0);
         sweep(at0, false, std::false_type());
         if (++l == k) return finish(at1);
     }

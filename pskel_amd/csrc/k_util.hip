@@ -145,17 +145,13 @@ hipError_t launch_fill_zero(void* dst, size_t bytes, hipStream_t st)
     return hipGetLastError();
 }
 
-// The widest unit that divides the row and both strides (the buffers are at
-// least 256-byte aligned).
+// Rows of bytes that are no multiple of 4 (others cross the link as they are).
 hipError_t launch_rows(void* dst, size_t dstride, const void* src, size_t sstride, size_t row_bytes, size_t rows,
                        hipStream_t st)
 {
     if (row_bytes == 0 || rows == 0) return hipSuccess;
-    const size_t a = row_bytes | dstride | sstride;
-    if (a % 16 == 0) return rows_launch<uint4>(dst, dstride, src, sstride, row_bytes, rows, st);
-    if (a % 8 == 0) return rows_launch<uint2>(dst, dstride, src, sstride, row_bytes, rows, st);
-    if (a % 4 == 0) return rows_launch<uint32_t>(dst, dstride, src, sstride, row_bytes, rows, st);
-    if (a % 2 == 0) return rows_launch<uint16_t>(dst, dstride, src, sstride, row_bytes, rows, st);
+    if ((row_bytes | dstride | sstride) % 2 == 0)
+        return rows_launch<uint16_t>(dst, dstride, src, sstride, row_bytes, rows, st);
     return rows_launch<uint8_t>(dst, dstride, src, sstride, row_bytes, rows, st);
 }
 

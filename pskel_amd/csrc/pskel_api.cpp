@@ -438,10 +438,7 @@ bool ends_single(const RunPlan& plan, const pskel_launch_cfg_t& cfg, size_t iter
 // 5-point 2048^2 147 -> 132, 331 -> 194.  A 2D launch of an
 // even number of sweeps writes a spare buffer; without one (odd2d) a launch
 // fuses one sweep less.
-// On register tiles the launch is as deep as rtile2d_plan makes it (*rt).  A run
-// that keeps the state before its last sweep (keep_prev) ends in a single sweep or,
-// where the kernel can store that state beside its own result, in an even launch
-// (50 sweeps of CLOUDSIM at 4096^2: 719 us, with that store 733).
+// On register tiles the launch is as deep as rtile2d_plan makes it (*rt).
 size_t next_k(const pskel::Grid& g, const RunPlan& plan, size_t done, size_t iterations, int kmax, size_t every,
               RtPlan* rt)
 {
@@ -452,8 +449,6 @@ size_t next_k(const pskel::Grid& g, const RunPlan& plan, size_t done, size_t ite
         if (g.ndim == 2 && !reduces && k > 1 && (done + k) % every == 0) k -= 1;
     }
     if (plan.rtile) {
-        const bool stores = plan.pattern == PAT_CLOUD || (every && (done + k) % every == 0);
-        if (plan.keep_prev && k > 1 && done + k == iterations && (!stores || k % 2 == 1)) k -= 1;
         *rt = plan.pattern == PAT_LIFE8 ? life_tiles_plan((int)g.W, (int)g.H, k, g.odd_2d_launches)
                                         : rtile2d_plan(plan.pattern, (int)g.W, (int)g.H, k, g.odd_2d_launches);
         return (size_t)rt->k;
@@ -464,9 +459,8 @@ size_t next_k(const pskel::Grid& g, const RunPlan& plan, size_t done, size_t ite
 
 // FP64 partials of the register-tile launches that end on a residual step: the
 // last of those that cover an interval, which are the same in every interval.
-size_t rtile2d_partials(const pskel::Grid& g, RunPlan plan, const pskel_launch_cfg_t& cfg)
+size_t rtile2d_partials(const pskel::Grid& g, const RunPlan& plan, const pskel_launch_cfg_t& cfg)
 {
-    plan.keep_prev = false;  // an interval that is not the run's last
     if (!plan.rtile || plan.pattern == PAT_LIFE8 || cfg.residual_every <= 0) return 0;
     const size_t every = (size_t)cfg.residual_every;
     const int W = (int)g.W, H = (int)g.H;
@@ -475,8 +469,6 @@ size_t rtile2d_partials(const pskel::Grid& g, RunPlan plan, const pskel_launch_c
         RtPlan q;
         for (size_t done = 0; done < every; done += (size_t)q.k) (void)next_k(g, plan, done, every, 1, every, &q);
         nb = rtile2d_blocks(W, H, q);
-        // with keep_prev the run's last interval ends the same way or in a single sweep
-        if (!g.odd_2d_launches) nb = std::max(nb, rtile2d_blocks(W, H, rtile2d_plan(plan.pattern, W, H, 1, false)));
     } else {  // any launch that may end a longer one
         for (size_t k = 1; k <= kRtMaxDepth; ++k) {
             const RtPlan q = rtile2d_plan(plan.pattern, W, H, k, g.odd_2d_launches);
@@ -494,12 +486,20 @@ size_t rtile2d_partials(const pskel::Grid& g, RunPlan plan, const pskel_launch_c
 // the old current becomes the spare.
 // Sweeps at range r keep r rows and columns at each edge and write the cells
 // inside them, so the spare goes on holding at most r of its ring.
-void pskel::advance_state(pskel::Grid& g, size_t k, int radius)
+// A launch that kept the state before its last sweep wrote that to the buffer of its
+// ring: the other one (even k), or, ring included, the spare, which changes places
+// with the state before the launch (odd k).
+void pskel::advance_state(pskel::Grid& g, size_t k, int radius, bool kept)
 {
     g.spare_width = std::min(g.spare_width, radius);
     if (k % 2 || g.ndim == 3) {
         std::swap(g.buf[0], g.buf[1]);
         g.parity ^= 1;
+        if (kept) {
+            std::swap(g.buf[1], g.buf[2]);
+            g.spare_parity = g.parity ^ 1;
+            g.spare_width = radius;
+        }
     } else {
         std::swap(g.buf[0], g.buf[2]);
         g.spare_parity = g.parity;
@@ -564,17 +564,16 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
         const void* src = g->buf[0];
         void* dst;
         const bool inplace = (k % 2) == 0 && ndim == 2;  // 3D writes every cell: no ring to keep
-        if (!inplace) {
-            dst = g->buf[1];
-        } else {
-            if (!g->buf[2]) return fail(PSKEL_ERR_RUNTIME, "spare buffer missing");
+        const bool kept = plan.keep_prev && k > 1 && done + k == iterations;
+        if ((inplace || kept) && !g->buf[2]) return fail(PSKEL_ERR_RUNTIME, "spare buffer missing");
+        if (inplace) {
             if (!spare_ring_ok(*g, plan.radius)) {
                 Sweep2D rs = make_sweep2d(g, g->buf[0], g->buf[2], nullptr, plan.radius);
                 PSKEL_HIP(launch_copy_ring2d(rs, g->elem, st));
                 spare_ring_copied(*g, plan.radius);
             }
-            dst = g->buf[2];
         }
+        dst = inplace ? g->buf[2] : g->buf[1];
         hipError_t e = hipSuccess;
         bool fused_res = false;
         const bool reduces = want_res && plan.rtile && plan.pattern != PAT_LIFE8;
@@ -594,7 +593,7 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
         }
         if (ndim == 2) {
             Sweep2D s = make_sweep2d(g, src, dst, g->buf[1], plan.radius);
-            if (plan.keep_prev && inplace && done + k == iterations) s.prev = g->buf[1];
+            if (kept) s.prev = inplace ? g->buf[1] : g->buf[2];
             const int bx = cfg.block_x > 0 ? cfg.block_x : 64;
             const int by = cfg.block_y > 0 ? cfg.block_y : 4;
             if (plan.pattern == PAT_CLOUD) {
@@ -652,7 +651,7 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
         }
         if (e != hipSuccess) return hip_fail(e, "stencil launch");
         nl++;
-        advance_state(*g, k, plan.radius);
+        advance_state(*g, k, plan.radius, kept);
         g->sweeps_done += k;
         if (want_res) {
             if (!fused_res) {
@@ -1293,8 +1292,9 @@ pskel_status_t pskel_run_iterative(pskel_grid_t* g, const pskel_stencil_desc_t* 
         for (size_t done = 0; done < iterations;) {
             RtPlan rt;
             const size_t k = next_k(*g, plan, done, iterations, kmax, every, &rt);
+            const bool kept = plan.keep_prev && k > 1 && done + k == iterations;
             if (k % 2 == 0 && g->ndim == 2) spare_ring_copied(*g, radius);  // ring copy in the graph
-            advance_state(*g, k, radius);
+            advance_state(*g, k, radius, kept);
             g->sweeps_done += k;
             done += k;
         }

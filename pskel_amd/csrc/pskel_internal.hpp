@@ -133,8 +133,9 @@ struct Grid {
     bool odd_2d_launches = false;  // 2D launches fuse an odd number of sweeps (no spare buffer)
 };
 
-// The ping-pong state after a launch of k sweeps at mask range `radius`.
-void advance_state(Grid& g, size_t k, int radius);
+// The ping-pong state after a launch of k sweeps at mask range `radius` (kept: which
+// also stored the state before its last sweep).
+void advance_state(Grid& g, size_t k, int radius, bool kept = false);
 
 // ---------------------------------------------------------------------------
 // Launch plumbing shared by the kernel TUs.
@@ -146,8 +147,7 @@ struct Sweep2D {
     int W, H;
     size_t pitch;
     int radius;
-    void* prev = nullptr;   // register tiles with partials or of CLOUDSIM, even depths: the state before
-                            // the last sweep goes here too
+    void* prev = nullptr;   // register and life tiles: the state before the last sweep goes here too
 };
 
 struct Sweep3D {

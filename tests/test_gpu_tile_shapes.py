@@ -77,7 +77,7 @@ def _inputs(pattern, shape):
     return a, b, None, lambda n: oracle.run_2d(s, a, n, out=b) if n else a
 
 
-def _job(bufs, pattern, a, b, winds, k):
+def _job(bufs, pattern, a, b, winds, k, keep=False):
     """the launch as a run issues it: odd k writes the other buffer, even k a spare"""
     j = shapes.Job()
     h, w = a.shape
@@ -86,6 +86,8 @@ def _job(bufs, pattern, a, b, winds, k):
     spare[1:-1, 1:w - 1] = 0  # the current state's ring, another interior
     j.src, j.ring = bufs.new(am), bufs.new(bm)
     j.dst = j.ring if k % 2 else bufs.new(spare)
+    if keep and k > 1:  # the state before the last sweep: the buffer of its ring, or any other
+        j.prev = bufs.new(np.zeros_like(am)) if k % 2 else j.ring
     j.pitch, j.W, j.H, j.pattern, j.k = am.shape[1], w, h, pattern, k
     if pattern == shapes.CLOUD:
         j.coeff = 0.01
@@ -111,22 +113,19 @@ def test_register_tile_shapes(gpu, pattern, r, nw):
     for shape in ((rows - 1, 94), (rows, 257), (rows + 1, 523), (3 * rows + 5, 1030)):
         a, b, winds, state = _inputs(pattern, shape)
         for k in (1, 2, 3, min(7, rows // 2 - 1), min(32, rows // 2 - 2)):
-            for residual in (False, True):
-                prev = k % 2 == 0 and (residual or pattern == shapes.CLOUD)
+            for residual, keep in ((False, False), (True, False), (False, True), (True, True)):
                 with _Buffers() as bufs:
-                    j, am = _job(bufs, pattern, a, b, winds, k)
+                    j, am = _job(bufs, pattern, a, b, winds, k, keep)
                     nb = l.shapes_rtile_blocks(shape[1], shape[0], r, nw, k)
                     part = np.full(nb, np.nan)
                     if residual:
                         j.partials = bufs.new(part)
-                    if prev:
-                        j.prev = j.ring
                     assert l.shapes_rtile(C.byref(j), r, nw) == 0, (shape, k)
                     L.check(L.lib().pskel_device_synchronize())
                     want, before = state(k), state(k - 1)
                     _same(bufs.read(j.dst, am), want, (shape, k, residual))
-                    if prev:
-                        _same(bufs.read(j.ring, am), before, (shape, k, residual, "prev"))
+                    if j.prev:
+                        _same(bufs.read(j.prev, am), before, (shape, k, residual, "prev"))
                     if residual:
                         total = bufs.read(j.partials, part).sum()
                         d = want.astype(np.float64) - before.astype(np.float64)
@@ -140,11 +139,14 @@ def test_life_tile_shapes(gpu, r, nw):
     for shape in ((rows - 1, 33), (rows, 2049), (rows + 1, 2078), (3 * rows + 5, 4100)):
         a, b, _, state = _inputs(shapes.LIFE8, shape)
         for k in (1, 2, min(7, rows // 2 - 1), min(30, rows // 2 - 2), min(31, rows // 2 - 1)):
-            with _Buffers() as bufs:
-                j, am = _job(bufs, shapes.LIFE8, a, b, None, k)
-                assert l.shapes_life(C.byref(j), r, nw) == 0, (shape, k)
-                L.check(L.lib().pskel_device_synchronize())
-                _same(bufs.read(j.dst, am), state(k), (shape, k))
+            for keep in (False, True):
+                with _Buffers() as bufs:
+                    j, am = _job(bufs, shapes.LIFE8, a, b, None, k, keep)
+                    assert l.shapes_life(C.byref(j), r, nw) == 0, (shape, k)
+                    L.check(L.lib().pskel_device_synchronize())
+                    _same(bufs.read(j.dst, am), state(k), (shape, k, keep))
+                    if j.prev:
+                        _same(bufs.read(j.prev, am), state(k - 1), (shape, k, "prev"))
 
 
 @pytest.mark.parametrize("pattern", [shapes.J5, shapes.BOX9])
