@@ -421,11 +421,10 @@ def measure_batch(steps, warmup, sweeps=200, compare=True, family_depths=None):
     """256 uneven grids, `sweeps` sweeps per step: persistent kernels per
     launch, captured in one hipGraph, with every grid's launch shape from the
     cost model at the family choices measured on the batch (tuner.batch.search,
-    timed here on the workload's own grids: life depth, f32 in LDS tiles or
-    through the register march); beside it the model's own picks, the same
-    batch at depth 1 (register tiles, the model's rows per lane) and the same
-    work launched grid by grid (one runIterativeGPU per grid, the reference's
-    way)."""
+    timed here on the workload's own grids: life depth, f32 one sweep or
+    fused); beside it the model's own picks, the same batch at depth 1 (the
+    model's rows per lane) and the same work launched grid by grid (one
+    runIterativeGPU per grid, the reference's way)."""
     from pskel_amd import api
     from pskel_amd import kernels as K
     from pskel_amd.tuner import batch as TB

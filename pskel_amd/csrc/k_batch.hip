@@ -105,7 +105,7 @@ __device__ __forceinline__ void run_ttile(const BatchEntry& E, const Sweep2D& s,
 
 // Work families, one kernel each so each keeps the registers its body needs
 // (one-sweep tiles, f32 LDS temporal tiles, bit-packed life tiles, f32 register
-// tiles of the 5-point and the 3x3 stencil, which need 79 and 91 registers, and
+// tiles of the 5-point and the 3x3 stencil, which need 76 and 88 registers, and
 // 130 in one kernel).
 enum BatchFamily : int { BF_REG = 0, BF_TTILE = 1, BF_BITS = 2, BF_J5 = 3, BF_BOX9 = 4, BF_COUNT = 5 };
 

@@ -24,7 +24,7 @@
 // cells.  Cells past the grid only ever reach ring cells.
 //
 // Measured, us per generation, against the bit tiles that ran before (a wave per
-// tile, at most 8 generations per launch): 8194^2 2.9 (9.7), 4096^2 1.6; 1000 x
+// tile, at most 8 generations per launch): 8194^2 2.8 (9.7), 4096^2 1.6; 1000 x
 // 1503 0.83 (3.6, one generation per launch).  The floor of an 8194^2 board is
 // 0.75 us of VALU; the rest is the halo (5 tiles of 1984 columns hold 4.1, 96 to
 // 104 of 128 rows are a tile's own) and the bytes of load and store.

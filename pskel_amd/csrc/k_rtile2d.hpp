@@ -27,9 +27,10 @@
 //
 // Measured, us per sweep, against the kernels that ran before (4 sweeps per
 // launch: LDS tiles or the register march; CLOUDSIM: one): 5-point 2048^2 1.6
-// (2.9), 4096^2 4.1 (7.1); 9-point 1021 x 1531 2.3 (3.4); CLOUDSIM 4096^2 14.2
-// (52), bound by the VALU (24 instructions per cell) and the 16 bytes per cell
-// and launch about equally.
+// (2.9), 4096^2 4.1 (7.1); 9-point 1021 x 1531 2.3 (3.4); CLOUDSIM 4096^2 14.7
+// (52; 14.4 without the state before the last sweep), bound by VALU issue (86% of
+// its rate, 31 instructions per cell for the formula's 24) and the 16 bytes per
+// cell and launch (69% of a copy's rate).
 #pragma once
 
 #include <type_traits>

@@ -6,8 +6,10 @@ the model's per-grid picks favour shallow launches; inside a batch's
 persistent launches that floor is shared and only the work counts.  So the
 family-wide choices are measured on the batch itself, the batch-level
 counterpart of the exhaustive search that judges the model: life at 1, 3, 5 or
-7 generations per launch, f32 at 1 or 3 sweeps (3 also by the name of the
-register march, which runs the same register tiles).  Every grid's tile at the chosen depth comes from the model.
+7 generations per launch, f32 at 1 or 3 sweeps (3 by the name of LDS tiles,
+which run where the batch finds them faster, or of the register march; both run
+register tiles elsewhere).  Every grid's tile at the chosen depth comes from the
+model.
 The timings run on scratch grids of the same shapes (the kernels' speed does
 not depend on the values), so the caller's grids are left as they are.  Above
 depth 1 the batch deepens a family's launches itself (pskel_batch_create), so
