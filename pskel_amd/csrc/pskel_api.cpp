@@ -590,6 +590,13 @@ pskel_status_t issue(pskel_grid_t* g, const pskel_stencil_desc_t& d, const Point
                 one.block_x = 0;
                 one.block_y = 0;
             }
+            if (plan.pattern == PAT_LIFE8) {
+                // short columns fill the device with waves: us a generation, (1, 4),
+                // (2, 4) and the default (4, 4): 200^2 3.1, 4.1, 6.1; 1000^2 3.3, 3.9,
+                // 5.4; 2000^2 4.9, 4.7, 5.9; 4000^2 10.5, 9.4, 9.7
+                one.tile_y = cells(g) < 3000000 ? 1 : 2;
+                one.tile_z = 4;
+            }
         }
         if (ndim == 2) {
             Sweep2D s = make_sweep2d(g, src, dst, g->buf[1], plan.radius);
