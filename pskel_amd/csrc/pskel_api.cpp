@@ -711,15 +711,22 @@ bool cloud_fields_fit(const pskel_grid_t* g)
 //   3000^2 1.18 and 1.12, 40000 x 300 1.16 and 1.13 (under 3M cells level or faster);
 //   CLOUDSIM, single sweeps: 9000 x 100, 3 sweeps 1.29 times slower, 100000 x 40
 //   67 / 137, 7 sweeps 154 / 219; 20000 x 40, 7 sweeps level, 40 1.16 times faster.
-// A residual step is reduced in the tiles' launch: there they win (0.4 to 0.85).
+// A residual step is reduced in the tiles' launch: there they win (0.4 to 0.85), but
+// for the 9-point stencil on those tall narrow grids every 8 sweeps or more: 16 rows,
+// us of 60 sweeps named / tiles, 20000 x 20 every 5, 8, 20: 425 / 330, 232 / 325,
+// 182 / 275; 11000 x 20 every 8 and 12 level, 20 1.18 times slower; 12000 x 110 still
+// 1.09 times faster every 8; 8 rows, 10000 x 20 every 8, 20: 178 / 209, 133 / 172.
 bool rtile_pays(int pattern, const pskel_grid_t* g, const pskel_launch_cfg_t& cfg, size_t iterations)
 {
     const size_t W = g->W, H = g->H, every = cfg.residual_every > 0 ? (size_t)cfg.residual_every : 0;
     const size_t run = every ? std::min(iterations, every) : iterations;  // sweeps that may share a launch
     if (pattern == PAT_CLOUD) return !((W <= 256 && H > 6000 && run <= 3) || (W <= 100 && H > 25000 && run < 8));
-    if (every && every <= iterations) return true;
-    if (cfg.tile_x != 0) return !(pattern == PAT_BOX9 && run <= 3 && (W * H >= 3000000 || H >= 20000));
     const size_t rows = cfg.tile_y > 0 ? (size_t)cfg.tile_y : 32;
+    if (every && every <= iterations) {
+        const size_t line = rows <= 8 && W <= 60 ? 9000 : (W <= 60 ? 700 : 850) * std::max<size_t>(rows, 16);
+        return !(pattern == PAT_BOX9 && cfg.tile_x == 0 && W <= 120 && H > line && every >= 8);
+    }
+    if (cfg.tile_x != 0) return !(pattern == PAT_BOX9 && run <= 3 && (W * H >= 3000000 || H >= 20000));
     if (pattern == PAT_BOX9 && W > 240 && W <= 360 && H >= 20000) return false;
     if (W > 120 || H <= 420 * rows) return true;
     return pattern == PAT_J5 && (run > 3 || W > 64 || rows > 16);

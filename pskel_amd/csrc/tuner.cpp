@@ -241,6 +241,15 @@ void features(const pskel_tune_query_t& q, const pskel_stencil_desc_t& d, const 
 }
 
 // Heuristic: the shapes the sweeps on MI355X found best for the large grids.
+// 9-point f32 grids that one column of LDS tiles (120 wide) covers run on those and not
+// on register tiles once they are this tall, and the rows of a tile decide their speed.
+// The shipped model, whose timings are of wider grids, names 64 rows there.
+bool tall_narrow9(const pskel_tune_query_t& q, const pskel_stencil_desc_t& d, int pat)
+{
+    return q.ndim == 2 && pat == PAT_BOX9 && q.storage == PSKEL_DTYPE_F32 && q.iterations >= 2 && q.width <= 120 &&
+           q.height > 3500 && desc_radius(d, 2) == 1;
+}
+
 pskel_launch_cfg_t heuristic(const pskel_tune_query_t& q, const pskel_stencil_desc_t& d)
 {
     const int pat = classify(d, q.ndim);
@@ -265,6 +274,13 @@ pskel_launch_cfg_t heuristic(const pskel_tune_query_t& q, const pskel_stencil_de
         const double cells = (double)q.width * q.height;
         if (q.iterations < 2) return tuned(0, 2, 4, 1);
         const int k = (int)std::min<size_t>(q.iterations, 4);
+        // us of 60 sweeps with tiles of 8, 16, 32 rows (64: register tiles), 20 columns:
+        // 10000 rows 100, 112, 144 (145); 20000: 185, 144, 183 (243); 30000: 236, 253,
+        // 221; 40000: 284, 290, 352, and of 120 columns 339, 321, 360
+        if (tall_narrow9(q, d, pat)) {
+            const auto h = q.height;
+            return tuned(0, h <= 14000 ? 8 : h > 24000 && h <= 32000 ? 32 : 16, 0, k);
+        }
         const double march_from = pat == PAT_J5 ? 0.9e6 : 4.0e6;
         if (cells >= march_from && march2d_fits_query(q) && desc_radius(d, 2) == 1) return tuned(4, 0, 0, k);
         return tuned(0, cells >= 0.8e6 ? 16 : 8, 0, k);
@@ -494,10 +510,10 @@ pskel_status_t pskel_tuner_choose(const pskel_mlp_t* model, const pskel_tune_que
         std::lock_guard<std::mutex> lock(g_predict_mutex);
         model = g_default_model;
     }
-    // the shipped model's training queries hold no field stencils and no masks
-    // without a specialised kernel; any other model's may
+    // the shipped model's training queries hold no field stencils, no masks without
+    // a specialised kernel and no tall narrow grids; any other model's may
     const int pat = classify(*d, q->ndim);
-    if (!model || (mlp_shipped(model) && (pat == PAT_GENERIC || pat == PAT_CLOUD))) {
+    if (!model || (mlp_shipped(model) && (pat == PAT_GENERIC || pat == PAT_CLOUD || tall_narrow9(*q, *d, pat)))) {
         *out = heuristic(*q, *d);
         return PSKEL_OK;
     }
