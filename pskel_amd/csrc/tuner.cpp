@@ -321,8 +321,16 @@ pskel_launch_cfg_t heuristic(const pskel_tune_query_t& q, const pskel_stencil_de
         return tuned(vd, rw, hs, 1);
     }
     // any other mask: the LDS tile (3D, 7 to 27 points: 2.5 to 10 times the plain
-    // kernel from 192 x 225 x 260 up, level with it or faster down to 60 x 70 x 50)
-    return tuned(0, 0, 0, 1);
+    // kernel from 192 x 225 x 260 up, level with it or faster down to 60 x 70 x 50);
+    // the plain kernel's block of four rows along w idles on grids thinner than that:
+    // 1000 x 1 x 1000, (64, 4) / (256, 1): 5.9 / 3.8 us; 1000 x 2 x 1000 with a halo,
+    // (64, 4), (128, 2), (256, 1): 14.5, 11.5, 12.2
+    pskel_launch_cfg_t c = tuned(0, 0, 0, 1);
+    if (q.ndim == 3 && q.width < 4 && q.depth >= 256) {
+        c.block_x = q.width == 2 ? 128 : 256;
+        c.block_y = q.width == 2 ? 2 : 1;
+    }
+    return c;
 }
 
 // ---------------------------------------------------------------------------
